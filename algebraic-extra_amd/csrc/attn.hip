@@ -84,6 +84,12 @@ int32_t check_aligned(const char* who, std::initializer_list<const void*> ptrs) 
   return 0;
 }
 
+// Row blocks of the backward pre-pass per (b, h), whichever the dtype.
+int sink_shares(int T, int D) {
+  if (T <= 0 || (D != 16 && D != 32 && D != 64)) return 0;
+  return pre_blocks(T, D, ALGX_F32);
+}
+
 int32_t check_shape(int B, int H, int T, int D, int dtype) {
   if (B < 0 || H < 0 || T < 0) return fail("attn: negative size");
   if (dtype != ALGX_BF16 && dtype != ALGX_F32) return fail("attn: dtype must be bf16 or f32");
@@ -197,7 +203,9 @@ extern "C" int64_t algx_attn_bwd_workspace_bytes(int32_t B, int32_t H, int32_t T
   const int64_t rows = (int64_t)B * H * T;
   const int64_t acc = rows * D * (int64_t)sizeof(float);
   const int64_t di = ((rows * (int64_t)sizeof(float) + 255) / 256) * 256;
-  return acc + di;
+  // the sink gradient's shares, one per row block of the pre-pass
+  const int64_t shares = (int64_t)B * H * sink_shares(T, D) * (int64_t)sizeof(float);
+  return acc + di + shares;
 }
 
 extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, const float* sink,
@@ -233,19 +241,24 @@ extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, co
   const bool mfma = mfma_supported(T, D, dtype) && !force_generic();
   float* dq_acc = (float*)workspace;
   float* di = (float*)((char*)workspace + rows * D * (int64_t)sizeof(float));
-  // The pre-pass forms di and dsink, and clears the dQ accumulator unless
-  // the forward already did (a workspace it prepared).
+  // The pre-pass forms di and the shares of dsink, and clears the dQ
+  // accumulator unless the forward already did (a workspace it prepared).
   const bool cleared = mfma && workspace_state == ALGX_ATTN_WS_CLEARED;
+  float* shares = (float*)((char*)di + ((rows * (int64_t)sizeof(float) + 255) / 256) * 256);
+  const SinkGrad sg{shares, sink != nullptr ? dsink : nullptr, pre_blocks(T, D, dtype), B, H};
   if (int32_t rc = launch_bwd_pre(dout, o, o_precise, stat, sink, di,
-                                  mfma && !cleared ? dq_acc : nullptr, dsink, B, H, T, D, dtype,
-                                  kl, kh, guard, s))
+                                  mfma && !cleared ? dq_acc : nullptr,
+                                  sg.dsink != nullptr ? shares : nullptr, B, H, T, D, dtype, kl,
+                                  kh, guard, s))
     return rc;
   if (mfma) {
     if (int32_t rc = launch_bwd_mfma(q, k, v, stat, di, dout, dq_acc, dk, dv, B, H, T, kl, kh,
                                      guard, s))
       return rc;
-    return launch_dq_finish(dq_acc, dq, rows * D, dtype, kl, kh, guard, q_scale, s);
+    return launch_dq_finish(dq_acc, dq, rows * D, dtype, kl, kh, guard, q_scale, sg, s);
   }
+  if (sg.dsink != nullptr)
+    if (int32_t rc = launch_sink_finish(sg, s)) return rc;
   if (int32_t rc = launch_bwd_generic(q, k, v, stat, di, dout, dq, dk, dv, B, H, T, D, dtype,
                                       q_scale, kl, guard, 1, s))
     return rc;

@@ -13,15 +13,27 @@ int32_t launch_prepare(const void* q, const void* k, const void* v, const float*
 // Guard word from `nblocks` triples of partial maxima (|q_s|^2, |k|^2, |v|).
 int32_t launch_guard_finish(const float* partial, int nblocks, const float* sink, int H,
                             float bound, float vmax, int32_t* guard, hipStream_t s);
-// Row pre-pass of the backward: di (and the sink gradient), and the dQ
+// The sink gradient's shares of the backward pre-pass (nblk per (b, h)) and
+// where their sums go; dsink null: no sink gradient.
+struct SinkGrad {
+  const float* part;
+  float* dsink;
+  int nblk, B, H;
+};
+// Row pre-pass of the backward: di (and, with a sink and sink_part, each
+// block's share of the sink gradient, pre_blocks() per (b, h)), and the dQ
 // accumulator cleared when dq_acc is given.
+int pre_blocks(int T, int D, int dtype);
 int32_t launch_bwd_pre(const void* dout, const void* o, const float* o_precise,
                        const float* stat, const float* sink, float* di, float* dq_acc,
-                       float* dsink, int B, int H, int T, int D, int dtype, const KVariant& low,
-                       const KVariant& high, const int32_t* guard, hipStream_t s);
+                       float* sink_part, int B, int H, int T, int D, int dtype,
+                       const KVariant& low, const KVariant& high, const int32_t* guard,
+                       hipStream_t s);
+// dsink from the shares, as a launch of its own or in the dQ finish.
+int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s);
 int32_t launch_dq_finish(const float* acc, void* dq, int64_t n, int dtype, const KVariant& low,
                          const KVariant& high, const int32_t* guard, float q_scale,
-                         hipStream_t s);
+                         const SinkGrad& sg, hipStream_t s);
 
 // Generic kernels: any T, D in {16, 32, 64}, bf16 or f32, every variant.
 int32_t launch_fwd_generic(const void* q_s, const void* k, const void* v, const float* sink,
