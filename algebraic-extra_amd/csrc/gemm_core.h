@@ -36,11 +36,17 @@ struct Operand {
   int K;
   // 0: plain row-major storage. Otherwise the operand is stored in blocks of
   // 32 contiguous columns of the row-major matrix ([cols / 32][rows][32],
-  // ld = 32) and bstride is the distance between blocks; the direct-to-LDS
-  // path reads it (whole 64-byte row pieces per 32-wide k stage), the
-  // register-staged path does not.
+  // ld = 32) and bstride is the distance between blocks (whole 64-byte row
+  // pieces per 32-wide k stage).
   int64_t bstride = 0;
 };
+
+// Elements between consecutive 32-wide k stages of an operand.
+template <bool KC>
+__device__ __forceinline__ int64_t kstep(const Operand& op) {
+  if (KC) return op.bstride ? op.bstride : BK;  // the next 32-column block
+  return (int64_t)BK * op.ld;                    // the next 32 rows
+}
 
 // Stages one 256 x 64 (mn x k) tile of an operand into registers (zero
 // outside): four 16-byte loads per thread.
@@ -66,8 +72,9 @@ struct TileAddr {
         const int kg = tid / (BM / 8), mg = tid % (BM / 8);
         const int mm = mn0 + 8 * mg;
         koff[c] = kChunks * kg + c;
+        const int64_t at = op.bstride ? (int64_t)(mm >> 5) * op.bstride + (mm & 31) : mm;
         mn_in[c] = mm < op.rows;
-        base[c] = op.p + (mn_in[c] ? (int64_t)koff[c] * op.ld + mm : 0);
+        base[c] = op.p + (mn_in[c] ? (int64_t)koff[c] * op.ld + at : 0);
       }
     }
   }
@@ -81,7 +88,7 @@ struct TileLoader {
   // is replaced by zeros when stored, so no wait for the load sits here.
   __device__ __forceinline__ void load(const Operand& op, const TileAddr<KC>& ad, int k0) {
     ok = 0;
-    const int64_t step = KC ? (int64_t)k0 : (int64_t)k0 * op.ld;
+    const int64_t step = (k0 / BK) * kstep<KC>(op);
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
       const bool in = ad.mn_in[c] && k0 + ad.koff[c] < op.K;
@@ -240,13 +247,6 @@ __device__ __forceinline__ const bf16* dma_src(const Operand& op, int mn0, int b
     const int64_t at = op.bstride ? (int64_t)(col >> 5) * op.bstride + (col & 31) : col;
     return col < op.rows ? op.p + (int64_t)r * op.ld + at : op.p;
   }
-}
-
-// Elements between consecutive 32-wide k stages of an operand.
-template <bool KC>
-__device__ __forceinline__ int64_t kstep(const Operand& op) {
-  if (KC) return op.bstride ? op.bstride : BK;  // the next 32-column block
-  return (int64_t)BK * op.ld;                    // the next 32 rows
 }
 
 // Bytes from op.p to the end of the last 16-byte piece the direct-to-LDS
@@ -558,6 +558,45 @@ __device__ __forceinline__ void gemm_tile_dma(const Operand& A, const Operand& B
   Acc out;
   gemm_seq_dma<AKC, BKC>(A, B, m0, 1, n0, ring, out, tid,
                          [&](int, int, Acc& a) { acc = a; });
+}
+
+// Product of one output tile over the k stages [st0, st1) of its operands:
+// the whole stages on the direct-to-LDS ring, then a partial last stage (K not
+// a multiple of BK) through registers, zero past K. The partial stage costs
+// one exposed memory round trip per tile; running every stage through
+// registers for its sake took the head's dh/dE launch 996 us at N = 4096,
+// d = 768, V = 33713, against 401 us so.
+template <bool AKC, bool BKC>
+__device__ __forceinline__ void gemm_tile_range(const Operand& A, const Operand& B, int m0, int n0,
+                                                int st0, int st1, const DmaRing& ring, Acc& acc,
+                                                int tid) {
+  Operand a = A, b = B;
+  a.p += st0 * kstep<AKC>(A);
+  b.p += st0 * kstep<BKC>(B);
+  const int k = min(A.K, st1 * BK) - st0 * BK, whole = k / BK * BK;
+  a.K = b.K = whole;
+  if (whole > 0)
+    gemm_tile_dma<AKC, BKC>(a, b, m0, n0, ring, acc, tid);
+  else
+    acc.zero();
+  if (whole < k) {
+    static_assert(kStageElems <= 2 * kDmaOpElems, "a register-staged operand stage fits a ring slot");
+    const int w = tid >> 6, lane = tid & 63;
+    a.K = b.K = k;
+    TileAddr<AKC> aa;
+    TileAddr<BKC> ab;
+    TileLoader<AKC> la;
+    TileLoader<BKC> lb;
+    aa.init(a, m0, tid);
+    ab.init(b, n0, tid);
+    la.load(a, aa, whole);
+    lb.load(b, ab, whole);
+    __syncthreads();  // the ring's last operand reads are done
+    la.store(ring.slot[0], tid);
+    lb.store(ring.slot[1], tid);
+    __syncthreads();
+    mma_stage<AKC, BKC>(ring.slot[0], ring.slot[1], acc, w / NWN, w % NWN, lane);
+  }
 }
 
 // LDS of a kernel built on the GEMM cores (DMA: a compile-time bool in

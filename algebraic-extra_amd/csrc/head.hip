@@ -342,54 +342,147 @@ struct GemmJob {
   int tiles_n;  // output tiles along n
 };
 
-template <bool AKC, bool BKC, typename TOut, bool ACCUM, bool DMA>
-__device__ __forceinline__ void gemm_job(const GemmJob& jb, int tile, bf16* lds,
-                                         const DmaRing& ring, int tid) {
+// acc of tile (m0, n0) into C; v(i, j, r) gives its values.
+template <typename TOut, bool ACCUM, typename Val>
+__device__ __forceinline__ void put_tile(const GemmJob& jb, int m0, int n0, int i, int j, int tid,
+                                         Val&& v) {
   const int w = tid >> 6, lane = tid & 63, g = lane >> 5, c32 = lane & 31;
   const int wm = w / NWN, wn = w % NWN;
+  const int n = n0 + WTN * wn + 32 * j + c32;
+  if (n >= jb.N) return;
+  TOut* C = reinterpret_cast<TOut*>(jb.C);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int m = m0 + WTM * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
+    if (m >= jb.M) continue;
+    TOut* dst = C + (int64_t)m * jb.ldc + n;
+    if (ACCUM)
+      *dst = from_f<TOut>(to_f(*dst) + v(r));
+    else
+      *dst = from_f<TOut>(v(r));
+  }
+}
+
+// A unit's float32 sums of a tile in the workspace, in the accumulators'
+// order: run q (4 values) of block (i, j) of thread tid is one 16-byte piece.
+constexpr int kSlotElems = BM * BN;
+__device__ __forceinline__ int64_t slot_at(int i, int j, int q, int tid) {
+  return ((int64_t)((i * TJ + j) * 4 + q) * kThreads + tid) * 4;
+}
+
+// K stages [st0, st1) of one output tile; slot null: written to C, else the
+// float32 sums go to the slot.
+template <bool AKC, bool BKC, typename TOut, bool ACCUM, bool DMA>
+__device__ __forceinline__ void gemm_job(const GemmJob& jb, int tile, int st0, int st1,
+                                         float* slot, bf16* lds, const DmaRing& ring, int tid) {
   const int m0 = (tile / jb.tiles_n) * BM, n0 = (tile % jb.tiles_n) * BN;
   Acc acc;
   if (DMA)
-    gemm_tile_dma<AKC, BKC>(jb.A, jb.B, m0, n0, ring, acc, tid);
+    gemm_tile_range<AKC, BKC>(jb.A, jb.B, m0, n0, st0, st1, ring, acc, tid);
   else
     gemm_tile<AKC, BKC>(jb.A, jb.B, m0, n0, lds, lds + 2 * kStageElems, acc, tid);
-  TOut* C = reinterpret_cast<TOut*>(jb.C);
+  if (DMA && slot != nullptr) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<f32x4*>(slot + slot_at(i, j, q, tid)) =
+              f32x4{acc.v[i][j][4 * q], acc.v[i][j][4 * q + 1], acc.v[i][j][4 * q + 2],
+                    acc.v[i][j][4 * q + 3]};
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-      const int n = n0 + WTN * wn + 32 * j + c32;
-      if (n >= jb.N) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + WTM * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
-        if (m >= jb.M) continue;
-        TOut* dst = C + (int64_t)m * jb.ldc + n;
-        if (ACCUM)
-          *dst = from_f<TOut>(to_f(*dst) + acc.v[i][j][r]);
-        else
-          *dst = from_f<TOut>(acc.v[i][j][r]);
-      }
-    }
+    for (int j = 0; j < TJ; ++j)
+      put_tile<TOut, ACCUM>(jb, m0, n0, i, j, tid, [&](int r) { return acc.v[i][j][r]; });
 }
 
-// The backward's two products of a token chunk in one launch (the long-K dh
-// tiles first): dh[t][c] = sum_v dz[t][v] E[v][c] in the first dh_slots
-// workgroups (n_dh tiles; dh_slots is n_dh rounded up to a multiple of 8),
-// then dE[v][c] (+)= sum_t dz[t][v] h[t][c].
-template <bool ACCUM, bool DMA>
-__global__ __launch_bounds__(kThreads) void head_grad_kernel(GemmJob dh, GemmJob de, int n_dh,
-                                                             int dh_slots, int n_de) {
-  GEMM_LDS_STAGES;
-  const int b = blockIdx.x;
-  if (b < dh_slots) {
-    if (b < n_dh)
-      gemm_job<true, false, bf16, false, DMA>(dh, xcd_tile(b, n_dh, dh.tiles_n), s0, ring,
-                                              threadIdx.x);
-  } else {
-    gemm_job<false, false, float, ACCUM, DMA>(de, xcd_tile(b - dh_slots, n_de, de.tiles_n), s0,
-                                              ring, threadIdx.x);
+// How the backward's two products are dealt to workgroups (grad_plan): every
+// dh tile in s1 chunks of c1 k stages, the first n_de - n_tail dE tiles whole
+// and the last n_tail in s2 chunks of c2. Chunked tiles leave float32 slots
+// (dh's first) that head_grad_finish adds in chunk order.
+struct GradPlan {
+  int n_dh, n_de, n_tail;
+  int s1, c1, s2, c2;
+  int dh_slots;  // workgroups per dh chunk: n_dh rounded up to a multiple of 8
+  int de_slots;  // workgroups of the whole dE tiles, rounded up alike
+  int64_t slots() const {
+    return (s1 > 1 ? (int64_t)s1 * n_dh : 0) + (s2 > 1 ? (int64_t)s2 * n_tail : 0);
   }
+};
+
+// The backward's two products of a token chunk in one launch (the long-K dh
+// tiles first): dh[t][c] = sum_v dz[t][v] E[v][c], then
+// dE[v][c] (+)= sum_t dz[t][v] h[t][c].
+template <bool ACCUM, bool DMA>
+__global__ __launch_bounds__(kThreads) void head_grad_kernel(GemmJob dh, GemmJob de, GradPlan pl,
+                                                             float* slots) {
+  GEMM_LDS_STAGES;
+  int b = blockIdx.x;
+  const int ndh = pl.s1 * pl.dh_slots;
+  if (b < ndh) {
+    const int chunk = b / pl.dh_slots, t = b % pl.dh_slots;
+    if (t >= pl.n_dh) return;
+    const int tile = xcd_tile(t, pl.n_dh, dh.tiles_n);
+    const int stages = (dh.A.K + BK - 1) / BK;
+    float* slot = pl.s1 > 1 ? slots + ((int64_t)chunk * pl.n_dh + tile) * kSlotElems : nullptr;
+    gemm_job<true, false, bf16, false, DMA>(dh, tile, chunk * pl.c1,
+                                            min(stages, (chunk + 1) * pl.c1), slot, s0, ring,
+                                            threadIdx.x);
+    return;
+  }
+  b -= ndh;
+  const int stages = (de.A.K + BK - 1) / BK, n_whole = pl.n_de - pl.n_tail;
+  int tile = 0, st0 = 0, st1 = stages;
+  float* slot = nullptr;
+  if (b < pl.de_slots) {
+    if (b >= n_whole) return;
+    tile = xcd_tile(b, n_whole, de.tiles_n);
+  } else {
+    b -= pl.de_slots;
+    const int chunk = b / pl.n_tail, t = b % pl.n_tail;
+    tile = n_whole + t;
+    if (pl.s2 > 1) {
+      st0 = chunk * pl.c2;
+      st1 = min(stages, st0 + pl.c2);
+      slot = slots + ((pl.s1 > 1 ? (int64_t)pl.s1 * pl.n_dh : 0) + (int64_t)chunk * pl.n_tail + t) *
+                         kSlotElems;
+    }
+  }
+  gemm_job<false, false, float, ACCUM, DMA>(de, tile, st0, st1, slot, s0, ring, threadIdx.x);
+}
+
+// Chunked tiles from their slots, added in chunk order. Block (tile, i * TJ + j)
+// takes one 32 x 32 block per wave; dh's tiles come first.
+template <bool ACCUM>
+__global__ __launch_bounds__(kThreads) void head_grad_finish(GemmJob dh, GemmJob de, GradPlan pl,
+                                                             const float* __restrict__ slots) {
+  const int n_first = pl.s1 > 1 ? pl.n_dh : 0;
+  const int tid = threadIdx.x, ij = blockIdx.y, i = ij / TJ, j = ij % TJ;
+  const bool is_dh = (int)blockIdx.x < n_first;
+  const int t = is_dh ? blockIdx.x : blockIdx.x - n_first;
+  const int n = is_dh ? pl.n_dh : pl.n_tail, s = is_dh ? pl.s1 : pl.s2;
+  const float* p = slots + ((is_dh ? 0 : (int64_t)pl.s1 * n_first) + t) * kSlotElems;
+  f32x4 v[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const f32x4*>(p + slot_at(i, j, q, tid));
+  for (int c = 1; c < s; ++c)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 u =
+          *reinterpret_cast<const f32x4*>(p + (int64_t)c * n * kSlotElems + slot_at(i, j, q, tid));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[q][e] += u[e];
+    }
+  auto val = [&](int r) { return v[r >> 2][r & 3]; };
+  const int tile = is_dh ? t : pl.n_de - pl.n_tail + t;
+  if (is_dh)
+    put_tile<bf16, false>(dh, tile / dh.tiles_n * BM, tile % dh.tiles_n * BN, i, j, tid, val);
+  else
+    put_tile<float, ACCUM>(de, tile / de.tiles_n * BM, tile % de.tiles_n * BN, i, j, tid, val);
 }
 
 int64_t vpad_of(int V) { return ((int64_t)V + BM - 1) / BM * BM; }
@@ -408,6 +501,71 @@ int chunk_tokens(int N, int V) {
   c = c / BN * BN;
   if (c < BN) c = BN;
   return (int)(c > N ? ((N + BN - 1) / BN) * BN : c);
+}
+
+// Deals the dh and dE tiles of a chunk of ntok tokens. `share` is one compute
+// unit's equal part of all k stages. A dh tile runs V / 32 stages, so few
+// tokens leave most of the chip idle behind a handful of long tiles: they are
+// cut into chunks of at most a share (of 16 stages at least: below that the
+// 256 KB a chunk leaves in memory costs more than its products). At
+// N = 1024, d = 384, V = 32768 (8 dh tiles of 1024 stages) the launch took
+// 600 us whole and 72 us in 16 chunks, plus 9 us for adding the slots. With
+// many tokens the last dE tiles would run as a partly filled round of whole
+// tiles: the ones that no longer fit into a share are cut in chunks of at
+// least 128 stages (a chunk's slot, written and read again, costs about 25
+// stages): 3116 us whole, 2838 + 7 us so at N = 16384, d = 1024, V = 50304.
+GradPlan grad_plan(int ntok, int d, int V, bool dma) {
+  constexpr int kUnits = 256;
+  GradPlan pl{};
+  const int tn = (d + BN - 1) / BN;
+  const int k1 = (V + BK - 1) / BK, k2 = (ntok + BK - 1) / BK;
+  pl.n_dh = (ntok + BM - 1) / BM * tn;
+  pl.n_de = (V + BM - 1) / BM * tn;
+  pl.s1 = pl.s2 = 1;
+  pl.c1 = k1;
+  pl.c2 = k2;
+  if (dma) {
+    const int64_t total = (int64_t)pl.n_dh * k1 + (int64_t)pl.n_de * k2;
+    const int share = (int)((total + kUnits - 1) / kUnits);
+    const int want = share > 16 ? share : 16;
+    if (k1 > want) {
+      pl.c1 = want;
+      pl.s1 = (k1 + want - 1) / want;
+      pl.c1 = (k1 + pl.s1 - 1) / pl.s1;
+      pl.s1 = (k1 + pl.c1 - 1) / pl.c1;
+    }
+    // Whole dE tiles that fit beside the dh units within a share.
+    const int64_t units = (int64_t)pl.s1 * pl.n_dh;
+    const int64_t rounds = units / kUnits, more = units % kUnits;
+    auto fit = [&](int64_t busy) { return busy >= share ? 0 : (share - busy) / k2; };
+    const int64_t room =
+        more * fit((rounds + 1) * pl.c1) + (kUnits - more) * fit(rounds * pl.c1);
+    if (k2 >= 256 && room < pl.n_de && room >= kUnits) {
+      pl.n_tail = pl.n_de - (int)(room / tn * tn);
+      pl.s2 = k2 / 128 < 4 ? k2 / 128 : 4;
+      pl.c2 = (k2 + pl.s2 - 1) / pl.s2;
+    }
+  }
+  pl.dh_slots = (pl.n_dh + 7) / 8 * 8;
+  pl.de_slots = (pl.n_de - pl.n_tail + 7) / 8 * 8;
+  return pl;
+}
+
+// dz of a chunk in 32-column blocks ([v / 32][t][32]), read direct-to-LDS by
+// the dh/dE launch: dh's 32-wide k stage reads one 64-byte piece per token
+// row, dE's reads 32 token rows of one block contiguously (2 KB), instead of
+// half lines of 100 KB rows. Needs the operands within the loads' 32-bit
+// offsets; else dz is row-major and the launch register-staged.
+bool grad_dma(int ntok, int d, int V) {
+  const int64_t blk = (int64_t)32 * ntok;
+  return dma_span_ok(Operand{nullptr, 32, ntok, V, blk}, true) &&
+         dma_span_ok(Operand{nullptr, 32, V, ntok, blk}, false) &&
+         dma_span_ok(Operand{nullptr, d, d, V}, false) &&
+         dma_span_ok(Operand{nullptr, d, d, ntok}, false);
+}
+
+int64_t grad_slot_bytes(int ntok, int d, int V) {
+  return grad_plan(ntok, d, V, grad_dma(ntok, d, V)).slots() * kSlotElems * (int64_t)sizeof(float);
 }
 
 int32_t check_head(const void* h, const void* E, const int32_t* targets, int N, int d, int V,
@@ -528,10 +686,15 @@ extern "C" int32_t algx_head_fwd(const void* h, const void* E, const int32_t* ta
 }
 
 extern "C" int64_t algx_head_bwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype) {
-  (void)d;
   if (N <= 0 || V <= 0) return 0;
   if (dtype == ALGX_F32) return head_f32_bwd_workspace(N, V);
-  return (int64_t)chunk_tokens(N, V) * vpad_of(V) * 2;
+  const int csize = chunk_tokens(N, V);
+  const int64_t dz = (int64_t)csize * vpad_of(V) * 2;
+  if (d <= 0) return dz;
+  // the slots of the full token chunks and of the last one
+  const int first = csize < N ? csize : N, last = N - (N - 1) / csize * csize;
+  const int64_t sf = grad_slot_bytes(first, d, V), sl = grad_slot_bytes(last, d, V);
+  return dz + (sf > sl ? sf : sl);
 }
 
 extern "C" int32_t algx_head_bwd(const void* h, const void* E, const int32_t* targets,
@@ -552,22 +715,14 @@ extern "C" int32_t algx_head_bwd(const void* h, const void* E, const int32_t* ta
   const int64_t ldz = vpad_of(V);
   const int csize = chunk_tokens(N, V);
   bf16* dz = (bf16*)workspace;
+  float* slots = (float*)((char*)workspace + (int64_t)csize * ldz * 2);
   const bf16* hb = (const bf16*)h;
   const bf16* eb = (const bf16*)E;
   for (int tok0 = 0; tok0 < N; tok0 += csize) {
     const int ntok = min(csize, N - tok0);
     const int ct = chunk_tiles_of(ntok, V);
-    // LDS-DMA stages in the dh/dE launch when both products have whole k
-    // stages (V and the chunk's token count multiples of BK). dz is then
-    // stored in 32-column blocks ([v / 32][t][32]): dh's 32-wide k stage
-    // reads one 64-byte piece per token row, dE's reads 32 token rows of one
-    // block contiguously (2 KB), instead of half lines of 100 KB rows.
     const int64_t blk = (int64_t)32 * ntok;
-    const bool dma = V % BK == 0 && ntok % BK == 0 &&
-                     dma_span_ok(Operand{nullptr, 32, ntok, V, blk}, true) &&
-                     dma_span_ok(Operand{nullptr, 32, V, ntok, blk}, false) &&
-                     dma_span_ok(Operand{nullptr, d, d, V}, false) &&
-                     dma_span_ok(Operand{nullptr, d, d, ntok}, false);
+    const bool dma = grad_dma(ntok, d, V);
     const int64_t bstride = dma ? blk : 0;
     dim3 gdz((ntok + BN - 1) / BN, ((V + BM - 1) / BM + ct - 1) / ct);
     launch_k(probe_for(ALGX_PROBE_HEAD_DZ),
@@ -583,14 +738,19 @@ extern "C" int32_t algx_head_bwd(const void* h, const void* E, const int32_t* ta
     const GemmJob jdh{dz_t, Operand{eb, d, d, V}, (bf16*)dh + (int64_t)tok0 * d, (int64_t)d,
                       ntok, d, tn};
     const GemmJob jde{dz_v, Operand{hb + (int64_t)tok0 * d, d, d, ntok}, dE, (int64_t)d, V, d, tn};
-    const int n_dh = ((ntok + BM - 1) / BM) * tn;
-    const int n_de = ((V + BM - 1) / BM) * tn;
-    const int dh_slots = (n_dh + 7) / 8 * 8;
+    const GradPlan pl = grad_plan(ntok, d, V, dma);
     auto gk = dma ? (tok0 == 0 ? head_grad_kernel<false, true> : head_grad_kernel<true, true>)
                   : (tok0 == 0 ? head_grad_kernel<false, false> : head_grad_kernel<true, false>);
-    launch_k(probe_for(ALGX_PROBE_HEAD_DE), gk, dim3(dh_slots + n_de), dim3(kThreads), s, jdh, jde,
-             n_dh, dh_slots, n_de);
+    const int grid = pl.s1 * pl.dh_slots + pl.de_slots + pl.s2 * pl.n_tail;
+    launch_k(probe_for(ALGX_PROBE_HEAD_DE), gk, dim3(grid), dim3(kThreads), s, jdh, jde, pl, slots);
     if (int32_t rc = check_launch("head_grad")) return rc;
+    const int nsplit = (pl.s1 > 1 ? pl.n_dh : 0) + (pl.s2 > 1 ? pl.n_tail : 0);
+    if (nsplit > 0) {
+      auto fk = tok0 == 0 ? head_grad_finish<false> : head_grad_finish<true>;
+      launch_k(Probe{}, fk, dim3(nsplit, TI * TJ), dim3(kThreads), s, jdh, jde, pl,
+               (const float*)slots);
+      if (int32_t rc = check_launch("head_grad_finish")) return rc;
+    }
   }
   return 0;
 }

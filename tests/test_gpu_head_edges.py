@@ -1,0 +1,62 @@
+"""The fused head's backward where its two products are cut into chunks:
+dh over the vocabulary, the last dE tiles over the tokens.
+
+References: the CPU oracle, and at the benchmark's size dense float64 math on
+the GPU. Tolerances as in test_gpu_qknorm_head.py.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from _tol import assert_bf16, rel_l2, to_np
+from algebraic_amd.kernels import fused_head
+from oracle import head as OH
+from test_gpu_qknorm_head import _head_inputs, _head_run
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("N,d,V", [(1, 64, 513), (31, 128, 1025), (33, 256, 4097),
+                                   (40, 264, 2047), (257, 128, 8191), (128, 384, 5074)])
+def test_chunked_backward_ragged_k(N, d, V):
+    """Vocabularies and token counts that are no multiple of the 32-wide k
+    stage (a chunk's last stage partial, or its only one), one to many dh
+    chunks, one to three output tiles along the width."""
+    h, e, t = _head_inputs(N, d, V, N + V, 0.2)
+    for kind, n, c in (("alg_ce", 8, 2.0), ("ce", 16, 16.0)):
+        got = _head_run(h, e, t, kind=kind, n=n, c=c, block_n=N)
+        (obj, tel), (dh, de) = OH.fused_head(to_np(h), to_np(e), to_np(t), kind=kind, n=n, c=c,
+                                             dtype="bf16", g_obj=1.0)
+        assert abs(got[0] - obj) <= 2e-4 + 2e-3 * abs(obj)
+        np.testing.assert_allclose(got[1], tel, rtol=2e-2, atol=2e-4)
+        assert_bf16(got[2], dh, what="dh")
+        assert rel_l2(got[3], de) <= 1e-2
+
+
+@pytest.mark.parametrize("chunk_mib", [0, 830])
+def test_chunked_backward_at_benchmark_size(monkeypatch, chunk_mib):
+    """N=16384, d=768, V=50304: dh whole, the last dE tiles in chunks; and the
+    same as two token chunks of 8192 (830 MiB of dz), where dh is cut as well
+    and the second launch adds its chunked dE tiles to the first's."""
+    if chunk_mib:
+        monkeypatch.setenv("ALGX_HEAD_CHUNK_BYTES", str(chunk_mib << 20))
+    N, d, V = 16384, 768, 50304
+    gen = torch.Generator(device=DEV).manual_seed(23)
+    h = torch.randn((N, d), device=DEV, generator=gen).bfloat16().requires_grad_(True)
+    e = (0.02 * torch.randn((V, d), device=DEV, generator=gen)).bfloat16().requires_grad_(True)
+    t = torch.randint(0, V, (N,), device=DEV, generator=gen)
+    obj, tel = fused_head(h, e, t, kind="ce")
+    dh, de = torch.autograd.grad(obj, [h, e])
+    with torch.no_grad():
+        h64, e64 = h.double(), e.double()
+        z = h64 @ e64.T
+        lse = torch.logsumexp(z, -1, keepdim=True)
+        nll = (lse - z.gather(1, t[:, None]))[:, 0]
+        dz = torch.exp(z - lse)
+        dz[torch.arange(N, device=DEV), t] -= 1.0
+        dz /= N
+        assert rel_l2(tel, nll) <= 1e-4
+        assert rel_l2(dh, dz @ e64) <= 1e-2
+        assert rel_l2(de, dz.T @ h64) <= 1e-2
