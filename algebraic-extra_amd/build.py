@@ -26,6 +26,8 @@ ARCH = "gfx950"
 EXTRA = {
     "attn_fwd_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attn_bwd_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attn_fwd_ragged.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attn_bwd_ragged.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "head.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_batched.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }

@@ -1,6 +1,6 @@
 // C ABI of the attention kernels: argument validation, variant conversion
-// and dispatch between the MFMA path (bf16, D=64, T%128==0) and the generic
-// path (everything else). A guarded MFMA call launches one kernel that reads
+// and dispatch between the MFMA path (bf16, D=64) and the generic path
+// (everything else). A guarded MFMA call launches one kernel that reads
 // the device guard word and runs the low or the high variant for the whole
 // grid; the generic path enqueues both variants and the unselected one
 // returns at once. Either way this mirrors lax.cond(in_range, low, high) of
@@ -71,6 +71,9 @@ int32_t scratch_on_current_device(float** out) {
   return 0;
 }
 
+// T in whole query blocks of the MFMA forward.
+bool whole_blocks(int T) { return acc_rows(T) == T; }
+
 bool force_generic() {
   const char* e = std::getenv("ALGX_FORCE_GENERIC");
   return e != nullptr && e[0] == '1';
@@ -82,6 +85,11 @@ int32_t check_aligned(const char* who, std::initializer_list<const void*> ptrs) 
     if (p != nullptr && (reinterpret_cast<uintptr_t>(p) & 15) != 0)
       return fail(std::string(who) + ": q, k, v, o, dO and gradient tensors must be 16-byte aligned");
   return 0;
+}
+
+// Bytes of the backward's dQ accumulator, which its workspace starts with.
+int64_t acc_bytes(int B, int H, int T, int D) {
+  return (int64_t)B * H * acc_rows(T) * D * (int64_t)sizeof(float);
 }
 
 // Row blocks of the backward pre-pass per (b, h), whichever the dtype.
@@ -180,13 +188,20 @@ extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v
   if (int32_t rc = check_aligned("attn_forward", {q, k, v, q_s, o, o_precise, bwd_workspace}))
     return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (mfma_supported(T, D, dtype) && !force_generic()) {
-    if (guard != nullptr && workspace == nullptr)
-      return fail("attn_forward: the guard needs the workspace");
+  // A guarded call without a workspace for the partial maxima takes the
+  // generic path where T is no multiple of the MFMA path's query block.
+  const bool mfma = mfma_supported(T, D, dtype) && !force_generic();
+  const bool parts = guard == nullptr || workspace != nullptr;
+  if (mfma && (parts || whole_blocks(T))) {
+    if (!parts) return fail("attn_forward: the guard needs the workspace");
     // The backward workspace starts with its float32 dQ accumulator.
     return launch_fwd_fused(q, k, v, sink, q_s, o, o_precise, stat, guard, (float*)workspace,
                             (float*)bwd_workspace, B, H, T, q_scale, bound, vmax, kl, kh, s);
   }
+  // The backward of such a call still runs MFMA and finds its accumulator
+  // cleared.
+  if (mfma && bwd_workspace != nullptr)
+    if (int32_t rc = fill_f32((float*)bwd_workspace, acc_bytes(B, H, T, D) / 4, 0.0f, s)) return rc;
   if (int32_t rc = launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound,
                                   vmax, s))
     return rc;
@@ -201,7 +216,7 @@ extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v
 
 extern "C" int64_t algx_attn_bwd_workspace_bytes(int32_t B, int32_t H, int32_t T, int32_t D) {
   const int64_t rows = (int64_t)B * H * T;
-  const int64_t acc = rows * D * (int64_t)sizeof(float);
+  const int64_t acc = acc_bytes(B, H, T, D);
   const int64_t di = ((rows * (int64_t)sizeof(float) + 255) / 256) * 256;
   // the sink gradient's shares, one per row block of the pre-pass
   const int64_t shares = (int64_t)B * H * sink_shares(T, D) * (int64_t)sizeof(float);
@@ -240,7 +255,7 @@ extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, co
     return rc;
   const bool mfma = mfma_supported(T, D, dtype) && !force_generic();
   float* dq_acc = (float*)workspace;
-  float* di = (float*)((char*)workspace + rows * D * (int64_t)sizeof(float));
+  float* di = (float*)((char*)workspace + acc_bytes(B, H, T, D));
   // The pre-pass forms di and the shares of dsink, and clears the dQ
   // accumulator unless the forward already did (a workspace it prepared).
   const bool cleared = mfma && workspace_state == ALGX_ATTN_WS_CLEARED;
@@ -255,7 +270,8 @@ extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, co
     if (int32_t rc = launch_bwd_mfma(q, k, v, stat, di, dout, dq_acc, dk, dv, B, H, T, kl, kh,
                                      guard, s))
       return rc;
-    return launch_dq_finish(dq_acc, dq, rows * D, dtype, kl, kh, guard, q_scale, sg, s);
+    return launch_dq_finish(dq_acc, dq, (int64_t)B * H, T, D, dtype, kl, kh, guard, q_scale, sg,
+                            s);
   }
   if (sg.dsink != nullptr)
     if (int32_t rc = launch_sink_finish(sg, s)) return rc;
@@ -279,9 +295,10 @@ extern "C" int32_t algx_attn_forward_noalloc(const void* q, const void* k, const
                                              float vmax, const algx_attn_variant* low,
                                              const algx_attn_variant* high, void* stream) {
   if (int32_t rc = check_shape(B, H, T, D, dtype)) return rc;
-  // The limit is checked for every guarded call, whichever path would run,
-  // before anything touches the device.
-  if (guard != nullptr && fwd_fused_partials(B, H, T) > kNoAllocParts)
+  // The limit is checked before anything touches the device, whichever path
+  // would run; it counts whole query blocks (a call with a partial last block
+  // and more partials than the scratch holds takes the generic path).
+  if (guard != nullptr && fwd_fused_partials(B, H, T / 128 * 128) > kNoAllocParts)
     return fail("attn_forward_noalloc: B * H * T / 128 exceeds the scratch limit of 65536 "
                 "forward workgroups; use algx_attn_forward with a workspace");
   if ((int64_t)B * H * T > 0 && (q == nullptr || k == nullptr || v == nullptr ||
@@ -289,7 +306,7 @@ extern "C" int32_t algx_attn_forward_noalloc(const void* q, const void* k, const
     return fail("attn_forward_noalloc: null pointer");
   float* part = nullptr;
   if (guard != nullptr && (int64_t)B * H * T > 0 && mfma_supported(T, D, dtype) &&
-      !force_generic()) {
+      !force_generic() && fwd_fused_partials(B, H, T) <= kNoAllocParts) {
     if (int32_t rc = scratch_on_current_device(&part)) return rc;
   }
   return algx_attn_forward(q, k, v, sink, q_s, o, o_precise, stat, guard, part, bwd_workspace, B,

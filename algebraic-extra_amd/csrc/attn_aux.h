@@ -31,9 +31,9 @@ int32_t launch_bwd_pre(const void* dout, const void* o, const float* o_precise,
                        hipStream_t s);
 // dsink from the shares, as a launch of its own or in the dQ finish.
 int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s);
-int32_t launch_dq_finish(const float* acc, void* dq, int64_t n, int dtype, const KVariant& low,
-                         const KVariant& high, const int32_t* guard, float q_scale,
-                         const SinkGrad& sg, hipStream_t s);
+int32_t launch_dq_finish(const float* acc, void* dq, int64_t heads, int T, int D, int dtype,
+                         const KVariant& low, const KVariant& high, const int32_t* guard,
+                         float q_scale, const SinkGrad& sg, hipStream_t s);
 
 // Generic kernels: any T, D in {16, 32, 64}, bf16 or f32, every variant.
 int32_t launch_fwd_generic(const void* q_s, const void* k, const void* v, const float* sink,
@@ -46,8 +46,12 @@ int32_t launch_bwd_generic(const void* q, const void* k, const void* v, const fl
                            const KVariant& var, const int32_t* guard, int want_low,
                            hipStream_t s);
 
-// MFMA kernels: bf16, D = 64, T % 128 == 0.
+// MFMA kernels: bf16, D = 64, any T.
 bool mfma_supported(int T, int D, int dtype);
+// Rows per head of the MFMA backward's float32 dQ accumulator: T rounded up to
+// whole 128-row query blocks, so that the forward clears and the backward adds
+// whole blocks.
+__host__ __device__ inline int acc_rows(int T) { return (T + 127) / 128 * 128; }
 // One launch per call: with a guard word the kernel runs `lo` or `hi` for the
 // whole grid; without one it runs `lo`.
 int32_t launch_fwd_mfma(const void* q_s, const void* k, const void* v, const float* sink,
@@ -70,5 +74,21 @@ int32_t launch_bwd_mfma(const void* q_s, const void* k, const void* v, const flo
                         const float* di, const void* dout, float* dq_acc, void* dk, void* dv,
                         int B, int H, int T, const KVariant& lo, const KVariant& hi,
                         const int32_t* guard, hipStream_t s);
+
+// The same launches for T that is no multiple of 128 (translation units of
+// their own).
+int32_t launch_fwd_ragged(const void* q_s, const void* k, const void* v, const float* sink,
+                          void* o, float* o_precise, float* stat, int B, int H, int T,
+                          const KVariant& lo, const KVariant& hi, const int32_t* guard,
+                          hipStream_t s);
+int32_t launch_fused_ragged(const void* q, const void* k, const void* v, const float* sink,
+                            void* q_s, void* o, float* o_precise, float* stat, int32_t* guard,
+                            float* partial, float* dq_zero, int B, int H, int T, float q_scale,
+                            float bound, float vmax, const KVariant& lo, const KVariant& hi,
+                            hipStream_t s);
+int32_t launch_bwd_ragged(const void* q, const void* k, const void* v, const float* stat,
+                          const float* di, const void* dout, float* dq_acc, void* dk, void* dv,
+                          int B, int H, int T, const KVariant& lo, const KVariant& hi,
+                          const int32_t* guard, hipStream_t s);
 
 }  // namespace algx

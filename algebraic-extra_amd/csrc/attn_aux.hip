@@ -192,9 +192,10 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(
       if (has_sink) ds_acc += sink_grad_term(var, b, stat[row], acc);
     }
     if (dq_acc != nullptr) {
+      const int64_t aoff = ((int64_t)bh * acc_rows(T_) + t) * D + sub * EPL;
       f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int i = 0; i < EPL; i += 4) *reinterpret_cast<f32x4*>(dq_acc + off + i) = z;
+      for (int i = 0; i < EPL; i += 4) *reinterpret_cast<f32x4*>(dq_acc + aoff + i) = z;
     }
   }
   if (has_sink && sink_part != nullptr) {
@@ -231,10 +232,12 @@ __global__ __launch_bounds__(256) void sink_finish_kernel(const float* __restric
 
 // dq = cast(cast(acc * slope) * q_scale): the kernel's dQ output rounding
 // (flash.py:592) followed by the VJP of the query pre-scale (flash.py:833).
-// With a sink, the first sg.H blocks sum its gradient instead (one head each).
+// acc holds pad more elements per head of `per_head` than dq does. With a
+// sink, the first sg.H blocks sum its gradient instead (one head each).
 template <typename T>
 __global__ __launch_bounds__(256) void dq_finish_kernel(const float* __restrict__ acc,
                                                         T* __restrict__ dq, int64_t n,
+                                                        int64_t per_head, int64_t pad,
                                                         KVariant low, KVariant high,
                                                         const int32_t* __restrict__ guard,
                                                         float q_scale, SinkGrad sg) {
@@ -248,7 +251,8 @@ __global__ __launch_bounds__(256) void dq_finish_kernel(const float* __restrict_
   int64_t i = ((int64_t)(blockIdx.x - nsink) * blockDim.x + threadIdx.x) * 4;
   const int64_t stride = (int64_t)(gridDim.x - nsink) * blockDim.x * 4;
   for (; i < n; i += stride) {
-    f32x4 a = *reinterpret_cast<const f32x4*>(acc + i);
+    const int64_t at = pad != 0 ? i + i / per_head * pad : i;
+    f32x4 a = *reinterpret_cast<const f32x4*>(acc + at);
 #pragma unroll
     for (int j = 0; j < 4; ++j) dq[i + j] = from_f<T>(round_to<T>(a[j] * slope) * q_scale);
   }
@@ -350,19 +354,21 @@ int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s) {
   return check_launch("attn_sink_finish");
 }
 
-int32_t launch_dq_finish(const float* acc, void* dq, int64_t n, int dtype, const KVariant& low,
-                         const KVariant& high, const int32_t* guard, float q_scale,
-                         const SinkGrad& sg, hipStream_t s) {
+int32_t launch_dq_finish(const float* acc, void* dq, int64_t heads, int T, int D, int dtype,
+                         const KVariant& low, const KVariant& high, const int32_t* guard,
+                         float q_scale, const SinkGrad& sg, hipStream_t s) {
+  const int64_t per_head = (int64_t)T * D, n = heads * per_head;
+  const int64_t pad = (int64_t)(acc_rows(T) - T) * D;
   int64_t nb = (n / 4 + 255) / 256;
   if (nb > 8192) nb = 8192;
   if (nb < 1) nb = 1;
   if (sg.dsink != nullptr) nb += sg.H;
   if (dtype == ALGX_BF16)
-    dq_finish_kernel<bf16><<<(int)nb, 256, 0, s>>>(acc, (bf16*)dq, n, low, high, guard, q_scale,
-                                                   sg);
+    dq_finish_kernel<bf16><<<(int)nb, 256, 0, s>>>(acc, (bf16*)dq, n, per_head, pad, low, high,
+                                                   guard, q_scale, sg);
   else
-    dq_finish_kernel<float><<<(int)nb, 256, 0, s>>>(acc, (float*)dq, n, low, high, guard, q_scale,
-                                                    sg);
+    dq_finish_kernel<float><<<(int)nb, 256, 0, s>>>(acc, (float*)dq, n, per_head, pad, low, high,
+                                                    guard, q_scale, sg);
   return check_launch("attn_dq_finish");
 }
 

@@ -142,10 +142,11 @@ int32_t algx_attn_fwd(const void* q_s, const void* k, const void* v, const float
 
 /* algx_attn_forward = algx_attn_prepare + algx_attn_fwd in one call
  * (flash.py:823-856 as one unit): the pre-scale, the guard and the forward.
- * For bf16, D = 64, T % 128 == 0 the forward kernel reads the raw q itself,
- * writes q_s (for the backward) and, with a guard buffer, one triple of
- * partial guard maxima per workgroup into `workspace`
- * (algx_attn_forward_workspace_bytes; may be NULL when guard is NULL). A
+ * For bf16, D = 64 the forward kernel reads the raw q itself, writes q_s (for
+ * the backward) and, with a guard buffer, one triple of partial guard maxima
+ * per workgroup into `workspace` (algx_attn_forward_workspace_bytes; may be
+ * NULL when guard is NULL, or when T is no multiple of 128: such a guarded
+ * call without it takes the slower kernels of the other shapes). A
  * second launch reduces them to the guard word and, only when out of range,
  * recomputes the forward with `high`, completing lax.cond. Other shapes run
  * the two calls. bwd_workspace: NULL, or the algx_attn_bwd_workspace_bytes

@@ -7,6 +7,8 @@ and rows of terms formed from the storage dtype, as in test_gpu_attention.py.
 import pytest
 import torch
 
+from _tol import rel_l2
+from algebraic_amd.kernels import flash_attention
 from test_gpu_attention import _check_all, _oracle, _rand, _run
 
 pytestmark = pytest.mark.gpu
@@ -25,3 +27,47 @@ def test_sink_gradient_row_blocks(T, dtype):
     got = _run(q, k, v, g, sink, block=T, **kw)
     want, _ = _oracle(q, k, v, g, sink, dtype, **kw)
     _check_all(got, want, dtype)
+
+
+@pytest.mark.parametrize("T", [1, 2, 31, 33, 63, 65, 100, 127, 129, 191, 193, 255, 257, 333, 449])
+@pytest.mark.parametrize("kw", [dict(kind="asinh", n=16, c=8.0, range_guard=True),
+                                dict(kind="asinh", n=4, c=16.0, shift=True, fast_rho=True),
+                                dict(kind="asinh", n=16, c=16.0, shift=False),
+                                dict(kind="softmax")],
+                         ids=["guarded", "shift", "clamped", "softmax"])
+def test_mfma_any_length(T, kw):
+    """bf16, D = 64 at lengths that end inside a wave's 32 rows, a 64-row tile,
+    a 128-query or a 256-key block: rows past the end are read as row T - 1
+    and must reach no output. Several heads, so that a write past one head
+    would land in the next."""
+    shape = (2, 3, T, 64)
+    q, k, v, g = _rand(shape, 300 + T)
+    sink = torch.tensor([0.3, -0.7, 0.1]).reshape(1, 3, 1, 1) if T % 2 else None
+    got = _run(q, k, v, g, sink, block=T, **kw)
+    want, _ = _oracle(q, k, v, g, sink, "bf16", **kw)
+    _check_all(got, want, "bf16")
+
+
+@pytest.mark.parametrize("T", [129, 300])
+def test_mfma_any_length_out_of_range(T):
+    """The guard's high variant at a ragged length: scores far outside the
+    unshifted range, and a maximum that only the last row holds."""
+    shape = (1, 2, T, 64)
+    q, k, v, g = _rand(shape, 17)
+    q[:, :, -1] *= 200.0
+    k[:, :, -1] *= 200.0
+    kw = dict(kind="asinh", n=16, c=8.0, range_guard=True)
+    got = _run(q, k, v, g, None, block=T, **kw)
+    want, res = _oracle(q, k, v, g, None, "bf16", **kw)
+    _check_all(got, want, "bf16")
+
+
+def test_ragged_backward_twice():
+    """A second backward of one graph takes a raw workspace, whose accumulator
+    (whole 128-row blocks per head) the row pre-pass clears."""
+    q, k, v, g = (x.cuda().requires_grad_(True) for x in _rand((2, 3, 77, 64), 5))
+    o = flash_attention(q, k, v, block=77, kind="asinh", n=16, c=8.0, range_guard=True)
+    first = torch.autograd.grad(o, [q, k, v], g.detach(), retain_graph=True)
+    second = torch.autograd.grad(o, [q, k, v], g.detach())
+    for a, b in zip(first, second):
+        assert rel_l2(a, b) <= 1e-3     # dq: float32 atomics, rounded to bf16
