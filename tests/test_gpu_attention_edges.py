@@ -71,3 +71,46 @@ def test_ragged_backward_twice():
     second = torch.autograd.grad(o, [q, k, v], g.detach())
     for a, b in zip(first, second):
         assert rel_l2(a, b) <= 1e-3     # dq: float32 atomics, rounded to bf16
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 63, 65, 130])
+@pytest.mark.parametrize("kw", [dict(kind="asinh", n=16, c=8.0, range_guard=True),
+                                dict(kind="asinh", n=8, c=1.0, shift=True, fast_rho=False),
+                                dict(kind="softmax")], ids=["guarded", "shift", "softmax"])
+def test_generic_row_tiles(T, D, dtype, kw):
+    """The kernels for float32 and other head widths: one row, tile edges, fewer
+    16-row tiles than waves and more, with and without a sink. (bf16 at
+    D = 64 takes the bf16 MFMA kernels.)"""
+    shape = (2, 2, T, D)
+    q, k, v, g = _rand(shape, 500 + T + D, dtype=dtype)
+    sink = torch.tensor([0.3, -0.7]).reshape(1, 2, 1, 1) if (T + D) % 2 else None
+    got = _run(q, k, v, g, sink, block=T, **kw)
+    want, _ = _oracle(q, k, v, g, sink, dtype, **kw)
+    _check_all(got, want, dtype)
+
+
+@pytest.mark.parametrize("kw", [dict(kind="asinh", n=16, c=8.0, shift=False),
+                                dict(kind="softmax")], ids=["clamped", "softmax"])
+def test_generic_later_rows_stay_apart(kw):
+    """An infinity in a later row reaches no earlier one, also inside its
+    16-row tile: o up to a value row, dv and dk from a query row onwards."""
+    T, j = 40, 21
+    q, k, v, g = (x.cuda() for x in _rand((1, 1, T, 64), 9, dtype="f32"))
+    ref = [x.clone().requires_grad_() for x in (q, k, v)]
+    o_ref = flash_attention(*ref, block=T, **kw)
+    g_ref = torch.autograd.grad(o_ref, ref, g)
+    bad = v.clone()
+    bad[0, 0, j] = float("inf")
+    o = flash_attention(q, k, bad, block=T, **kw)
+    # such a tile is summed in another order: float32 rounding
+    assert rel_l2(o[0, 0, :j], o_ref[0, 0, :j]) <= 1e-6
+    assert not torch.isfinite(o[0, 0, j:]).any()
+    bad = g.clone()
+    bad[0, 0, j] = float("inf")
+    o = flash_attention(*ref, block=T, **kw)
+    dq, dk, dv = torch.autograd.grad(o, ref, bad)
+    assert rel_l2(dq[0, 0, :j], g_ref[0][0, 0, :j]) <= 1e-6
+    assert rel_l2(dv[0, 0, j + 1:], g_ref[2][0, 0, j + 1:]) <= 1e-6
+    assert rel_l2(dk[0, 0, j + 1:], g_ref[1][0, 0, j + 1:]) <= 1e-6
