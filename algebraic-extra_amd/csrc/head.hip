@@ -687,7 +687,7 @@ extern "C" int32_t algx_head_fwd(const void* h, const void* E, const int32_t* ta
 
 extern "C" int64_t algx_head_bwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype) {
   if (N <= 0 || V <= 0) return 0;
-  if (dtype == ALGX_F32) return head_f32_bwd_workspace(N, V);
+  if (dtype == ALGX_F32) return head_f32_bwd_workspace(N, d > 0 ? d : 0, V);
   const int csize = chunk_tokens(N, V);
   const int64_t dz = (int64_t)csize * vpad_of(V) * 2;
   if (d <= 0) return dz;

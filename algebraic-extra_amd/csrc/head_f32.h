@@ -7,7 +7,7 @@
 namespace algx {
 
 int64_t head_f32_fwd_workspace(int N, int V);
-int64_t head_f32_bwd_workspace(int N, int V);
+int64_t head_f32_bwd_workspace(int N, int d, int V);
 int32_t head_f32_fwd(const float* h, const float* E, const int32_t* targets, float* stat,
                      float* zt, float* partial, int N, int d, int V, int kind, int log2n,
                      float inv_c, float clamp, hipStream_t s);

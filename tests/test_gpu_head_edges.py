@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from _tol import assert_bf16, rel_l2, to_np
+from _tol import assert_bf16, assert_f32, rel_l2, to_np
 from algebraic_amd.kernels import fused_head
 from oracle import head as OH
 from test_gpu_qknorm_head import _head_inputs, _head_run
@@ -60,3 +60,23 @@ def test_chunked_backward_at_benchmark_size(monkeypatch, chunk_mib):
         assert rel_l2(tel, nll) <= 1e-4
         assert rel_l2(dh, dz @ e64) <= 1e-2
         assert rel_l2(de, dz.T @ h64) <= 1e-2
+
+
+@pytest.mark.parametrize("N,d,V", [(1, 4, 2), (5, 6, 131), (127, 36, 129), (129, 132, 1021),
+                                   (130, 128, 4097), (640, 20, 700)])
+def test_float32_head_tile_edges(N, d, V):
+    """float32: widths with and without whole 16-byte rows, extents around the
+    128-wide tiles and the 16-wide k stage, products cut along k (V = 4097,
+    N = 640) and whole."""
+    rng = np.random.default_rng(N + d + V)
+    h = torch.from_numpy(rng.standard_normal((N, d)).astype(np.float32))
+    e = torch.from_numpy((rng.standard_normal((V, d)) * 0.15).astype(np.float32))
+    t = torch.from_numpy(rng.integers(0, V, N).astype(np.int64))
+    for kind, n, c in (("alg_ce", 8, 2.0), ("ce", 16, 16.0)):
+        got = _head_run(h, e, t, kind=kind, n=n, c=c, block_n=N)
+        (obj, tel), (dh, de) = OH.fused_head(to_np(h), to_np(e), to_np(t), kind=kind, n=n, c=c,
+                                             dtype="f32", g_obj=1.0)
+        assert abs(got[0] - obj) <= 1e-5 * abs(obj) + 1e-6
+        assert_f32(got[1], tel, what="telemetry")
+        assert_f32(got[2], dh, what="dh")
+        assert_f32(got[3], de, what="dE")
