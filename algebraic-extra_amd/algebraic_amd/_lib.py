@@ -68,6 +68,9 @@ SIGNATURES = {
     "algx_head_fwd_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
     "algx_head_fwd": (_i32, [_p, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _f32, _f32,
                              _i32, _p]),
+    "algx_head_loss_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
+    "algx_head_loss": (_i32, [_p, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _f32, _f32,
+                              _i32, _p]),
     "algx_head_bwd_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
     "algx_head_bwd": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32,
                              _f32, _f32, _i32, _p]),

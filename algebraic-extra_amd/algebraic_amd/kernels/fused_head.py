@@ -31,30 +31,6 @@ def _root(value, n):
     return out
 
 
-def _ipow(x, n):
-    out, base = None, x
-    while n:
-        if n & 1:
-            out = base if out is None else out * base
-        n >>= 1
-        if n:
-            base = base * base
-    return out
-
-
-def _telemetry(stat, zt, kind, n, c, clamp):
-    """(per-token NLL or target probability, objective), fused_head.py:219-229."""
-    if kind == "ce":
-        nll = stat - zt
-        return nll, nll.mean()
-    x = torch.clamp(zt / c, max=clamp)
-    rad = 1.0 + x * x
-    t = x.abs() + rad * torch.rsqrt(rad)
-    rho = torch.where(x >= 0, t, 1.0 / t)
-    pt = _ipow(rho * stat, n)
-    return pt, (1.0 - pt).mean()
-
-
 class _HeadFn(torch.autograd.Function):
     """Custom VJP of fused_head.py:232-257 (residuals h, E, targets, stat)."""
 
@@ -64,15 +40,15 @@ class _HeadFn(torch.autograd.Function):
         V = embed.shape[0]
         e = embed.to(h.dtype).contiguous()                    # fused_head.py:168
         stat = torch.empty(N, dtype=torch.float32, device=h.device)
-        zt = torch.empty(N, dtype=torch.float32, device=h.device)
+        tel = torch.empty(N, dtype=torch.float32, device=h.device)
+        obj = torch.empty((), dtype=torch.float32, device=h.device)
         kcode = _lib.HEAD_CE if kind == "ce" else _lib.HEAD_ALG_CE
         dt = _lib.dtype_code(h.dtype)
-        ws = torch.empty(max(1, _lib.query("algx_head_fwd_workspace_bytes", N, d, V, dt)),
+        ws = torch.empty(_lib.query("algx_head_loss_workspace_bytes", N, d, V, dt),
                          dtype=torch.uint8, device=h.device)
-        _lib.call("algx_head_fwd", _lib.ptr(h), _lib.ptr(e), _lib.ptr(targets), _lib.ptr(stat),
-                  _lib.ptr(zt), _lib.ptr(ws), N, d, V, kcode, int(n), float(1.0 / c),
-                  float(clamp), dt, _lib.stream())
-        tel, obj = _telemetry(stat, zt, kind, n, c, clamp)
+        _lib.call("algx_head_loss", _lib.ptr(h), _lib.ptr(e), _lib.ptr(targets), _lib.ptr(stat),
+                  _lib.ptr(tel), _lib.ptr(obj), _lib.ptr(ws), N, d, V, kcode, int(n),
+                  float(1.0 / c), float(clamp), dt, _lib.stream())
         ctx.cfg = (kind, n, c, clamp, embed.dtype)
         ctx.save_for_backward(h, e, targets, stat)
         ctx.mark_non_differentiable(tel)

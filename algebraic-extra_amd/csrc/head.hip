@@ -188,27 +188,98 @@ __global__ __launch_bounds__(kThreads) void head_fwd_kernel(
   }
 }
 
-// stat = m + log l (ce) or l^(-1/n) (alg_ce) from the chunk partials
-// (fused_head.py:113-116).
+// What the chunk partials of a token become. stat = m + log l (ce) or
+// l^(-1/n) (alg_ce) (fused_head.py:113-116); with tel, also the per-token NLL
+// or target probability and the block's share of the objective
+// (fused_head.py:219-229).
+struct HeadStat {
+  const float* partial;
+  const int32_t* targets;
+  float* zt;        // target logits; a target outside the vocabulary reads 0
+  float* stat;
+  float* tel;       // null: stat and zt only
+  float* obj_part;  // one share per block
+  int nchunks, N, V, log2n;
+  float inv_c, clamp;
+};
+
+// A workgroup takes 64 tokens, its four waves every fourth chunk each: few
+// tokens come with many chunks, and one thread per token walked them serially
+// on a handful of CUs (18 us at N = 1024 with 64 chunks, now 4.5 us).
+constexpr int kStatTokens = 64;
+
 template <int KIND>
-__global__ __launch_bounds__(256) void head_stat_kernel(const float* __restrict__ partial,
-                                                        int nchunks, int N, int log2n,
-                                                        float* __restrict__ stat) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= N) return;
+__global__ __launch_bounds__(256) void head_stat_kernel(HeadStat p) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  constexpr float kLog2e = 1.4426950408889634f;
+  __shared__ float red_m[4][kStatTokens], red_l[4][kStatTokens];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = blockIdx.x * kStatTokens + lane;
   float m = -1e30f, l = 0.0f;
-  for (int c = 0; c < nchunks; ++c) {
-    const float mc = partial[((int64_t)c * N + t) * 2 + 0];
-    const float lc = partial[((int64_t)c * N + t) * 2 + 1];
+  auto merge = [&](float mo, float lo) {
     if (KIND == ALGX_HEAD_CE) {
-      const float mm = __builtin_fmaxf(m, mc);
-      l = l * __expf(m - mm) + lc * __expf(mc - mm);
+      const float mm = __builtin_fmaxf(m, mo);
+      l = l * __builtin_amdgcn_exp2f((m - mm) * kLog2e) +
+          lo * __builtin_amdgcn_exp2f((mo - mm) * kLog2e);
       m = mm;
     } else {
-      l += lc;
+      l += lo;
+    }
+  };
+  if (t < p.N) {
+#pragma unroll 4
+    for (int c = w; c < p.nchunks; c += 4) {
+      const f32x2 x = *reinterpret_cast<const f32x2*>(p.partial + ((int64_t)c * p.N + t) * 2);
+      merge(x[0], x[1]);
     }
   }
-  stat[t] = KIND == ALGX_HEAD_CE ? m + __logf(l) : inv_root(l, log2n);
+  red_m[w][lane] = m;
+  red_l[w][lane] = l;
+  __syncthreads();
+  if (w != 0) return;
+#pragma unroll
+  for (int ww = 1; ww < 4; ++ww) merge(red_m[ww][lane], red_l[ww][lane]);
+  float term = 0.0f;
+  if (t < p.N) {
+    const float st = KIND == ALGX_HEAD_CE ? m + __logf(l) : inv_root(l, p.log2n);
+    p.stat[t] = st;
+    const int tgt = p.targets[t];
+    float z = 0.0f;
+    if ((unsigned)tgt < (unsigned)p.V)
+      z = p.zt[t];
+    else
+      p.zt[t] = 0.0f;
+    if (p.tel != nullptr) {
+      float tel;
+      if (KIND == ALGX_HEAD_CE) {
+        tel = st - z;
+        term = tel;
+      } else {
+        const float x = __builtin_fminf(z * p.inv_c, p.clamp);
+        const float r = __builtin_fabsf(x) + __builtin_sqrtf(__builtin_fmaf(x, x, 1.0f));
+        tel = pow2n((x >= 0.0f ? r : 1.0f / r) * st, p.log2n);
+        term = 1.0f - tel;
+      }
+      p.tel[t] = tel;
+    }
+  }
+  if (p.tel == nullptr) return;
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) term += __shfl_xor(term, s, 64);
+  if (lane == 0) p.obj_part[blockIdx.x] = term;
+}
+
+// obj = the mean over the tokens from the blocks' shares.
+__global__ __launch_bounds__(256) void head_mean_kernel(const float* __restrict__ part, int nparts,
+                                                        int N, float* __restrict__ obj) {
+  __shared__ float red[4];
+  float s = 0.0f;
+  for (int i = threadIdx.x; i < nparts; i += 256) s += part[i];
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) obj[0] = ((red[0] + red[1]) + (red[2] + red[3])) / (float)N;
 }
 
 // dz tile of a token chunk: dz[t][v] = bf16(f(z) * scale), 0 for padded v.
@@ -645,11 +716,53 @@ int nchunks_of(int N, int V) {
 
 using namespace algx;
 
-extern "C" int64_t algx_head_fwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype) {
-  (void)d;
+namespace {
+
+int64_t fwd_partial_bytes(int32_t N, int32_t V, int32_t dtype) {
   if (N <= 0 || V <= 0) return 0;
   if (dtype == ALGX_F32) return head_f32_fwd_workspace(N, V);
   return (int64_t)nchunks_of(N, V) * N * 2 * sizeof(float);
+}
+
+int stat_blocks(int N) { return (N + kStatTokens - 1) / kStatTokens; }
+
+// The forward up to stat and zt, and with tel the telemetry and objective
+// (obj_part: stat_blocks(N) floats).
+int32_t head_forward(const void* h, const void* E, const int32_t* targets, float* stat, float* zt,
+                     float* tel, float* obj, float* partial, float* obj_part, int32_t N, int32_t d,
+                     int32_t V, int32_t kind, int32_t n, float inv_c, float clamp, int32_t dtype,
+                     hipStream_t s) {
+  const int log2n = kind == ALGX_HEAD_ALG_CE ? ilog2(n) : 0;
+  int nch;
+  if (dtype == ALGX_F32) {
+    if (int32_t rc = head_f32_fwd((const float*)h, (const float*)E, targets, zt, partial, N, d, V,
+                                  kind, log2n, inv_c, clamp, &nch, s))
+      return rc;
+  } else {
+    nch = nchunks_of(N, V);
+    dim3 grid((N + BN - 1) / BN, nch);
+    launch_k(probe_for(ALGX_PROBE_HEAD_FWD), pick_head_fwd(kind, log2n, d, V, N), grid,
+             dim3(kThreads), s, (const bf16*)h, (const bf16*)E, targets, zt, partial, N, d, V,
+             log2n, inv_c, clamp, chunk_tiles_of(N, V));
+    if (int32_t rc = check_launch("head_fwd")) return rc;
+  }
+  const HeadStat p{partial, targets, zt, stat, tel, obj_part, nch, N, V, log2n, inv_c, clamp};
+  const int nb = stat_blocks(N);
+  if (kind == ALGX_HEAD_CE)
+    head_stat_kernel<ALGX_HEAD_CE><<<nb, 256, 0, s>>>(p);
+  else
+    head_stat_kernel<ALGX_HEAD_ALG_CE><<<nb, 256, 0, s>>>(p);
+  if (int32_t rc = check_launch("head_stat")) return rc;
+  if (tel == nullptr) return 0;
+  head_mean_kernel<<<1, 256, 0, s>>>(obj_part, nb, N, obj);
+  return check_launch("head_mean");
+}
+
+}  // namespace
+
+extern "C" int64_t algx_head_fwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype) {
+  (void)d;
+  return fwd_partial_bytes(N, V, dtype);
 }
 
 extern "C" int32_t algx_head_fwd(const void* h, const void* E, const int32_t* targets,
@@ -659,30 +772,29 @@ extern "C" int32_t algx_head_fwd(const void* h, const void* E, const int32_t* ta
   if (int32_t rc = check_head(h, E, targets, N, d, V, kind, n, dtype)) return rc;
   if (N == 0) return 0;
   if (stat == nullptr || zt == nullptr || workspace == nullptr) return fail("head_fwd: null output");
-  hipStream_t s = (hipStream_t)stream;
-  const int nch = nchunks_of(N, V);
-  dim3 grid((N + BN - 1) / BN, nch);
-  const int log2n = kind == ALGX_HEAD_ALG_CE ? ilog2(n) : 0;
+  return head_forward(h, E, targets, stat, zt, nullptr, nullptr, (float*)workspace, nullptr, N, d,
+                      V, kind, n, inv_c, clamp, dtype, (hipStream_t)stream);
+}
+
+extern "C" int64_t algx_head_loss_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype) {
+  (void)d;
+  if (N <= 0 || V <= 0) return 0;
+  // the chunk partials, the target logits, the objective's shares
+  return fwd_partial_bytes(N, V, dtype) + ((int64_t)N + stat_blocks(N)) * (int64_t)sizeof(float);
+}
+
+extern "C" int32_t algx_head_loss(const void* h, const void* E, const int32_t* targets,
+                                  float* stat, float* tel, float* obj, void* workspace, int32_t N,
+                                  int32_t d, int32_t V, int32_t kind, int32_t n, float inv_c,
+                                  float clamp, int32_t dtype, void* stream) {
+  if (int32_t rc = check_head(h, E, targets, N, d, V, kind, n, dtype)) return rc;
+  if (N == 0) return fail("head_loss: the mean over no tokens");
+  if (stat == nullptr || tel == nullptr || obj == nullptr || workspace == nullptr)
+    return fail("head_loss: null output");
   float* partial = (float*)workspace;
-  // The target logit starts at 0 as in fused_head.py:80 (a target outside
-  // the vocabulary tiles is never met).
-  if (int32_t rc = fill_f32(zt, N, 0.0f, s)) return rc;
-  if (dtype == ALGX_F32)
-    return head_f32_fwd((const float*)h, (const float*)E, targets, stat, zt, partial, N, d, V,
-                        kind, log2n, inv_c, clamp, s);
-  {
-    const Probe probe = probe_for(ALGX_PROBE_HEAD_FWD);
-    launch_k(probe, pick_head_fwd(kind, log2n, d, V, N),
-             grid, dim3(kThreads), s, (const bf16*)h, (const bf16*)E, targets, zt, partial, N, d,
-             V, log2n, inv_c, clamp, chunk_tiles_of(N, V));
-  }
-  if (int32_t rc = check_launch("head_fwd")) return rc;
-  const int nb = (N + 255) / 256;
-  if (kind == ALGX_HEAD_CE)
-    head_stat_kernel<ALGX_HEAD_CE><<<nb, 256, 0, s>>>(partial, nch, N, log2n, stat);
-  else
-    head_stat_kernel<ALGX_HEAD_ALG_CE><<<nb, 256, 0, s>>>(partial, nch, N, log2n, stat);
-  return check_launch("head_stat");
+  float* zt = (float*)((char*)workspace + fwd_partial_bytes(N, V, dtype));
+  return head_forward(h, E, targets, stat, zt, tel, obj, partial, zt + N, N, d, V, kind, n, inv_c,
+                      clamp, dtype, (hipStream_t)stream);
 }
 
 extern "C" int64_t algx_head_bwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype) {

@@ -15,7 +15,7 @@
 //
 // Forward: grid (token tiles, vocabulary chunks); per-token online statistics
 // merged over the lanes and waves that share a token and written as
-// (chunk, token) partials for head_f32_stat_kernel. Backward: the logit
+// (chunk, token) partials for the head's statistics kernel. Backward: the logit
 // gradient dz (float32, [tokens][V rounded up to 128]) of a token chunk, then
 // the two products, each cut along k where its tiles alone would not fill the
 // chip.
@@ -260,28 +260,6 @@ __global__ __launch_bounds__(FTHR, 2) void head_f32_fwd_kernel(
   }
 }
 
-// stat = m + log l (ce) or l^(-1/n) (alg_ce) from the chunk partials.
-template <int KIND>
-__global__ __launch_bounds__(256) void head_f32_stat_kernel(const float* __restrict__ partial,
-                                                            int nchunks, int N, int log2n,
-                                                            float* __restrict__ stat) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= N) return;
-  float m = -1e30f, l = 0.0f;
-  for (int c = 0; c < nchunks; ++c) {
-    const float mc = partial[((int64_t)c * N + t) * 2 + 0];
-    const float lc = partial[((int64_t)c * N + t) * 2 + 1];
-    if (KIND == ALGX_HEAD_CE) {
-      const float mm = __builtin_fmaxf(m, mc);
-      l = l * __expf(m - mm) + lc * __expf(mc - mm);
-      m = mm;
-    } else {
-      l += lc;
-    }
-  }
-  stat[t] = KIND == ALGX_HEAD_CE ? m + __logf(l) : inv_root(l, log2n);
-}
-
 // dz[t][v] = f(z) * scale for the tokens [tok0, tok0 + ntok), 0 for v >= V
 // (fused_head.py:127-145 with dz in float32). Tokens on m, vocabulary on n:
 // 32 lanes store 32 consecutive columns.
@@ -419,10 +397,11 @@ bool vec_ok(int d, const void* h, const void* E) {
 
 int64_t head_f32_fwd_workspace(int N, int V) { return (int64_t)nchunks_f32(N, V) * N * 2 * 4; }
 
-int32_t head_f32_fwd(const float* h, const float* E, const int32_t* targets, float* stat,
-                     float* zt, float* partial, int N, int d, int V, int kind, int log2n,
-                     float inv_c, float clamp, hipStream_t s) {
+int32_t head_f32_fwd(const float* h, const float* E, const int32_t* targets, float* zt,
+                     float* partial, int N, int d, int V, int kind, int log2n, float inv_c,
+                     float clamp, int* nchunks, hipStream_t s) {
   const int nch = nchunks_f32(N, V);
+  *nchunks = nch;
   dim3 grid((N + FT - 1) / FT, nch);
   const bool vec = vec_ok(d, h, E);
   auto fn = kind == ALGX_HEAD_CE
@@ -431,13 +410,7 @@ int32_t head_f32_fwd(const float* h, const float* E, const int32_t* targets, flo
                        : head_f32_fwd_kernel<ALGX_HEAD_ALG_CE, false>);
   fn<<<grid, FTHR, 0, s>>>(h, E, targets, zt, partial, N, d, V, log2n, inv_c, clamp,
                            chunk_tiles_f32(N, V));
-  if (int32_t rc = check_launch("head_f32_fwd")) return rc;
-  const int nb = (N + 255) / 256;
-  if (kind == ALGX_HEAD_CE)
-    head_f32_stat_kernel<ALGX_HEAD_CE><<<nb, 256, 0, s>>>(partial, nch, N, log2n, stat);
-  else
-    head_f32_stat_kernel<ALGX_HEAD_ALG_CE><<<nb, 256, 0, s>>>(partial, nch, N, log2n, stat);
-  return check_launch("head_f32_stat");
+  return check_launch("head_f32_fwd");
 }
 
 // Tokens per backward chunk: the float32 dz scratch is capped at 2 GiB.

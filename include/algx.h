@@ -206,6 +206,14 @@ int64_t algx_head_fwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t d
 int32_t algx_head_fwd(const void* h, const void* E, const int32_t* targets, float* stat,
                       float* zt, void* workspace, int32_t N, int32_t d, int32_t V, int32_t kind,
                       int32_t n, float inv_c, float clamp, int32_t dtype, void* stream);
+/* algx_head_fwd and what fused_head.py:219-229 forms from it: tel float32 (N,),
+ * the per-token NLL (ce) or target probability (alg_ce), and obj, one float32,
+ * the mean of tel or of 1 - tel. N > 0. */
+int64_t algx_head_loss_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype);
+int32_t algx_head_loss(const void* h, const void* E, const int32_t* targets, float* stat,
+                       float* tel, float* obj, void* workspace, int32_t N, int32_t d, int32_t V,
+                       int32_t kind, int32_t n, float inv_c, float clamp, int32_t dtype,
+                       void* stream);
 int64_t algx_head_bwd_workspace_bytes(int32_t N, int32_t d, int32_t V, int32_t dtype);
 int32_t algx_head_bwd(const void* h, const void* E, const int32_t* targets, const float* stat,
                       const float* scale, void* dh, float* dE, void* workspace, int32_t N,

@@ -80,3 +80,24 @@ def test_float32_head_tile_edges(N, d, V):
         assert_f32(got[1], tel, what="telemetry")
         assert_f32(got[2], dh, what="dh")
         assert_f32(got[3], de, what="dE")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 320])
+def test_loss_over_token_blocks(N, dtype):
+    """Telemetry and objective around the statistics kernel's 64-token blocks,
+    with many chunks per token; a target outside the vocabulary has target
+    logit 0 (fused_head.py:80)."""
+    V, d = 3001, 64
+    h, e, t = _head_inputs(N, d, V, 3 + N, 0.2)
+    h = h if dtype == "bf16" else h.float()
+    t[0] = -1
+    t[N // 2] = V + 2
+    z = to_np(h) @ to_np(e.bfloat16() if dtype == "bf16" else e).T
+    lse = np.log(np.exp(z - z.max(-1, keepdims=True)).sum(-1)) + z.max(-1)
+    inside = (t.numpy() >= 0) & (t.numpy() < V)
+    zt = np.where(inside, z[np.arange(N), np.where(inside, t.numpy(), 0)], 0.0)
+    obj, tel = fused_head(h.to(DEV), e.to(DEV), t.to(DEV), kind="ce", block_n=N)
+    # float32 sums of 3001 terms: 1e-6 relative, and one rounding of lse - zt
+    np.testing.assert_allclose(to_np(tel), lse - zt, rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(float(obj), (lse - zt).mean(), rtol=1e-5)
