@@ -18,43 +18,13 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """Contiguous with a 16-byte aligned base (the kernels move 16-byte vectors)."""
     t = t.contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
-class _RMSNormFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, gain, eps):
-        D = x.shape[-1]
-        rows = x.numel() // D if D else 0
-        y = torch.empty_like(x)
-        _lib.call("algx_rms_norm_fwd", _lib.ptr(x), _lib.ptr(gain), _lib.ptr(y), rows, D,
-                  _lib.dtype_code(x.dtype), float(eps), _lib.stream())
-        ctx.eps = eps
-        ctx.save_for_backward(x, gain)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, gain = ctx.saved_tensors
-        D = x.shape[-1]
-        rows = x.numel() // D if D else 0
-        dt = _lib.dtype_code(x.dtype)
-        dy = _aligned(dy.to(x.dtype))
-        dx = torch.empty_like(x)
-        dgain = ws = None
-        if gain is not None:
-            dgain = torch.empty(D, dtype=torch.float32, device=x.device)
-            ws = torch.empty(max(1, _lib.query("algx_rms_norm_bwd_workspace_bytes", rows, D, dt)),
-                             dtype=torch.uint8, device=x.device)
-        _lib.call("algx_rms_norm_bwd", _lib.ptr(x), _lib.ptr(gain), _lib.ptr(dy), _lib.ptr(dx),
-                  _lib.ptr(dgain), _lib.ptr(ws), rows, D, dt, float(ctx.eps), _lib.stream())
-        return dx, dgain, None
 
 
 def rms_norm(x: torch.Tensor, gain: Optional[torch.Tensor], eps: float = 1e-5) -> torch.Tensor:
@@ -70,43 +40,7 @@ def rms_norm(x: torch.Tensor, gain: Optional[torch.Tensor], eps: float = 1e-5) -
         raise ValueError(f"gain must have shape ({D},)")
     if not eps > 0:
         raise ValueError("rms_norm epsilon must be positive")
-    if gain is None:
-        return _RMSNormFn.apply(_aligned(x), None, float(eps))
-    g32 = gain.to(torch.float32).contiguous()
-    return _RMSNormFn.apply(_aligned(x), g32, float(eps))
-
-
-class _AddRMSNormFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, r, gain, eps):
-        D = x.shape[-1]
-        rows = x.numel() // D if D else 0
-        xsum, y = torch.empty_like(x), torch.empty_like(x)
-        _lib.call("algx_add_rms_norm_fwd", _lib.ptr(x), _lib.ptr(r), _lib.ptr(gain),
-                  _lib.ptr(xsum), _lib.ptr(y), rows, D, _lib.dtype_code(x.dtype), float(eps),
-                  _lib.stream())
-        ctx.eps = eps
-        ctx.save_for_backward(xsum, gain)
-        return xsum, y
-
-    @staticmethod
-    def backward(ctx, dxsum, dy):
-        xsum, gain = ctx.saved_tensors
-        D = xsum.shape[-1]
-        rows = xsum.numel() // D if D else 0
-        dt = _lib.dtype_code(xsum.dtype)
-        dy = torch.zeros_like(xsum) if dy is None else _aligned(dy.to(xsum.dtype))
-        dres = torch.zeros_like(xsum) if dxsum is None else _aligned(dxsum.to(xsum.dtype))
-        dx = torch.empty_like(xsum)
-        dgain = ws = None
-        if gain is not None:
-            dgain = torch.empty(D, dtype=torch.float32, device=xsum.device)
-            ws = torch.empty(max(1, _lib.query("algx_rms_norm_bwd_workspace_bytes", rows, D, dt)),
-                             dtype=torch.uint8, device=xsum.device)
-        _lib.call("algx_add_rms_norm_bwd", _lib.ptr(xsum), _lib.ptr(gain), _lib.ptr(dy),
-                  _lib.ptr(dres), _lib.ptr(dx), _lib.ptr(dgain), _lib.ptr(ws), rows, D, dt,
-                  float(ctx.eps), _lib.stream())
-        return dx, dx, dgain, None
+    return _native.ops().rms_norm(x, gain, float(eps))
 
 
 def add_rms_norm(x: torch.Tensor, r: torch.Tensor, gain: Optional[torch.Tensor],
@@ -127,8 +61,7 @@ def add_rms_norm(x: torch.Tensor, r: torch.Tensor, gain: Optional[torch.Tensor],
         raise ValueError(f"gain must have shape ({D},)")
     if not eps > 0:
         raise ValueError("rms_norm epsilon must be positive")
-    g32 = None if gain is None else gain.to(torch.float32).contiguous()
-    return _AddRMSNormFn.apply(_aligned(x), _aligned(r), g32, float(eps))
+    return _native.ops().add_rms_norm(x, r, gain, float(eps))
 
 
 class _ALUFn(torch.autograd.Function):
@@ -192,32 +125,6 @@ def alu_glu(gate: torch.Tensor, up: torch.Tensor, beta: float = 1.0) -> torch.Te
     return _ALUGLUFn.apply(_aligned(gate), _aligned(up), float(beta))
 
 
-class _GLUPackedFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, gu, act, beta):
-        cols = gu.shape[-1] // 2
-        rows = gu.numel() // (2 * cols)
-        y = torch.empty(gu.shape[:-1] + (cols,), dtype=gu.dtype, device=gu.device)
-        code = _lib.GLU_ALU if act == "alu" else _lib.GLU_SILU
-        _lib.call("algx_glu_packed_fwd", _lib.ptr(gu), _lib.ptr(y), rows, cols, code,
-                  _lib.dtype_code(gu.dtype), float(beta), _lib.stream())
-        ctx.cfg = (code, beta)
-        ctx.save_for_backward(gu)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        (gu,) = ctx.saved_tensors
-        code, beta = ctx.cfg
-        cols = gu.shape[-1] // 2
-        rows = gu.numel() // (2 * cols)
-        dy = _aligned(dy.to(gu.dtype))
-        dgu = torch.empty_like(gu)
-        _lib.call("algx_glu_packed_bwd", _lib.ptr(gu), _lib.ptr(dy), _lib.ptr(dgu), rows, cols,
-                  code, _lib.dtype_code(gu.dtype), float(beta), _lib.stream())
-        return dgu, None, None
-
-
 def glu_packed(gu: torch.Tensor, act: str = "alu", beta: float = 1.0) -> torch.Tensor:
     """``gate * act(up)`` for ``gu = [gate | up]`` on the last axis (one GEMM
     against ``[w_g | w_u]``, model.py:184-191): ``act="alu"`` is
@@ -231,4 +138,5 @@ def glu_packed(gu: torch.Tensor, act: str = "alu", beta: float = 1.0) -> torch.T
     width = 8 if gu.dtype == torch.bfloat16 else 4
     if (gu.shape[-1] // 2) % width:
         raise NotImplementedError(f"glu_packed needs gate/up widths that are a multiple of {width}")
-    return _GLUPackedFn.apply(_aligned(gu), act, float(beta))
+    code = _lib.GLU_ALU if act == "alu" else _lib.GLU_SILU
+    return _native.ops().glu_packed(gu, code, float(beta))

@@ -24,12 +24,13 @@ elsewhere; the reference makes that choice once per Pallas score tile, the
 kernels here per score (the two agree to ~3e-5 relative).
 """
 
+import functools
 import math
 from typing import NamedTuple, Optional
 
 import torch
 
-from .. import _lib
+from .. import _lib, _native
 
 LANES = 128
 NEG = -1e4
@@ -100,80 +101,30 @@ def _c_variant(var: Variant) -> _lib.AttnVariant:
         clamp=float(var.clamp), poly_rho=int(var.poly_rho))
 
 
-class _Plan(NamedTuple):
-    low: Variant
-    high: Optional[Variant]      # set when the range guard dispatches
-    q_scale: float
-    bound: float
-    vmax: float
-    has_sink: bool
+def _fields(var: Variant):
+    """The fields of algx_attn_variant, in order."""
+    return (_lib.SOFTMAX if var.kind == "softmax" else _lib.ASINH, int(var.n), int(var.shift),
+            int(var.fast_rho), int(var.inv_stat), int(var.bounded_scores),
+            int(var.precise_output), float(var.clamp), int(var.poly_rho))
 
 
-class _FlashFn(torch.autograd.Function):
-    """Custom VJP of flash.py:708-729 (residuals q, k, v, sink, o, stat)."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, sink, plan: _Plan):
-        B, H, T, D = q.shape
-        dt = _lib.dtype_code(q.dtype)
-        dev = q.device
-        st = _lib.stream()
-        guard = None
-        if plan.high is not None:
-            words = _lib.query("algx_attn_guard_words")
-            guard = torch.empty(words, dtype=torch.int32, device=dev)
-        # One call: q_s = cast(q * scale) (flash.py:833), the guard word when
-        # guarded (:834-849) and the forward (:853-856).
-        q_s = torch.empty_like(q)
-        o = torch.empty_like(q)
-        stat = torch.empty((B, H, T), dtype=torch.float32, device=dev)
-        precise = plan.low.precise_output or (plan.high is not None and plan.high.precise_output)
-        o_precise = torch.empty(q.shape, dtype=torch.float32, device=dev) if precise else None
-        ws = None
-        if guard is not None:
-            ws = torch.empty(_lib.query("algx_attn_forward_workspace_bytes", B, H, T, D),
-                             dtype=torch.uint8, device=dev)
-        # When a backward will follow, its workspace is allocated here and
-        # prepared by the forward in passing (its dQ accumulator cleared).
-        bws = None
-        if any(ctx.needs_input_grad[:4]):
-            bws = torch.empty(_lib.query("algx_attn_bwd_workspace_bytes", B, H, T, D),
-                              dtype=torch.uint8, device=dev)
-        lo = _c_variant(plan.low)
-        hi = _c_variant(plan.high) if plan.high is not None else None
-        _lib.call("algx_attn_forward", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(sink),
-                  _lib.ptr(q_s), _lib.ptr(o), _lib.ptr(o_precise), _lib.ptr(stat),
-                  _lib.ptr(guard), _lib.ptr(ws), _lib.ptr(bws), B, H, T, D, dt, plan.q_scale,
-                  plan.bound, plan.vmax, lo, hi, st)
-        ctx.plan = plan
-        ctx.bws = bws
-        ctx.save_for_backward(q_s, k, v, sink, o, o_precise, stat, guard)
-        return o
-
-    @staticmethod
-    def backward(ctx, do):
-        q_s, k, v, sink, o, o_precise, stat, guard = ctx.saved_tensors
-        plan = ctx.plan
-        B, H, T, D = q_s.shape
-        dt = _lib.dtype_code(q_s.dtype)
-        do = do.to(q_s.dtype).contiguous()
-        dq, dk, dv = torch.empty_like(q_s), torch.empty_like(k), torch.empty_like(v)
-        dsink = torch.empty((H,), dtype=torch.float32, device=q_s.device) if sink is not None else None
-        # The forward's prepared workspace serves one backward; a second one
-        # (retain_graph) hands it over as raw memory.
-        ws, state = ctx.bws, _lib.ATTN_WS_CLEARED
-        ctx.bws = None
-        if ws is None:
-            ws = torch.empty(_lib.query("algx_attn_bwd_workspace_bytes", B, H, T, D),
-                             dtype=torch.uint8, device=q_s.device)
-            state = _lib.ATTN_WS_RAW
-        lo = _c_variant(plan.low)
-        hi = _c_variant(plan.high) if plan.high is not None else None
-        _lib.call("algx_attn_bwd", _lib.ptr(q_s), _lib.ptr(k), _lib.ptr(v), _lib.ptr(sink),
-                  _lib.ptr(o), _lib.ptr(o_precise), _lib.ptr(stat), _lib.ptr(do),
-                  _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(dsink), _lib.ptr(ws), state,
-                  B, H, T, D, dt, plan.q_scale, lo, hi, _lib.ptr(guard), _lib.stream())
-        return dq, dk, dv, dsink, None
+@functools.lru_cache(maxsize=256, typed=True)
+def _plan(kind, n, c, T, D, shift, fast_rho, inv_stat, compact_stat, poly_rho, range_guard,
+          has_sink):
+    """The call's variants, query scale and guard bounds, from its options
+    alone (flash.py:816-852)."""
+    var = make_variant(kind, n, c, T, shift, fast_rho, inv_stat, compact_stat, poly_rho)
+    scale = 1.0 / (math.sqrt(D) * c)    # c is 1 for softmax
+    if not (range_guard and kind == "asinh" and n <= 32):
+        return _native.ops().flash_plan(_fields(var), None, scale, 0.0, 0.0)
+    if poly_rho:
+        raise ValueError("range_guard is for exact radical evaluation")  # flash.py:835-836
+    bound = min(16.0, var.clamp / 2)
+    vmax = min(1e8, 1e37 / ((T + int(has_sink)) * (2 * bound + 1) ** n))
+    low = var._replace(shift=False, inv_stat=True, bounded_scores=True)
+    high = var._replace(shift=True, inv_stat=False, fast_rho=False, bounded_scores=False,
+                        head_resident=False, precise_output=True)
+    return _native.ops().flash_plan(_fields(low), _fields(high), scale, bound, vmax)
 
 
 def flash_attention(q, k, v, sink_logit: Optional[torch.Tensor] = None, *, kind: str = "softmax",
@@ -197,7 +148,7 @@ def flash_attention(q, k, v, sink_logit: Optional[torch.Tensor] = None, *, kind:
     bk = min(block_k or block, T)
     if T % bq or T % bk:
         raise ValueError(f"sequence length {T} must be divisible by blocks ({bq}, {bk})")
-    var = make_variant(kind, n, c, T, shift, fast_rho, inv_stat, compact_stat, poly_rho)
+    make_variant(kind, n, c, T, shift, fast_rho, inv_stat, compact_stat, poly_rho)
     bf16 = q.dtype == k.dtype == v.dtype == torch.bfloat16
     resident_supported = (T in (512, 1024, 2048) and D == 64 and bf16 and not poly_rho and
                           (kind == "softmax" or n == 16))
@@ -219,22 +170,13 @@ def flash_attention(q, k, v, sink_logit: Optional[torch.Tensor] = None, *, kind:
     if D not in (16, 32, 64):
         raise ValueError(f"head dimension {D} is not supported (16, 32 or 64)")
     unit = 1.0 if kind == "softmax" else float(c)
-    scale = 1.0 / (math.sqrt(D) * unit)
-    has_sink = sink_logit is not None
-    if has_sink:
+    plan = _plan(kind, n, unit, T, D, shift, fast_rho, inv_stat, compact_stat, poly_rho,
+                 range_guard, sink_logit is not None)
+    if (sink_logit is not None and
+            not (isinstance(sink_logit, torch.Tensor) and sink_logit.numel() == H and
+                 sink_logit.dtype == torch.float32 and sink_logit.device == q.device)):
+        # Any other form: one float32 logit per head first, in kernel units.
         sink_in = torch.as_tensor(sink_logit, device=q.device).to(torch.float32)
-        sink = (torch.broadcast_to(sink_in.reshape(-1), (H,)) / unit).contiguous()
-    else:
-        sink = None
-    if range_guard and kind == "asinh" and n <= 32:
-        if poly_rho:
-            raise ValueError("range_guard is for exact radical evaluation")  # flash.py:835-836
-        bound = min(16.0, var.clamp / 2)
-        vmax = min(1e8, 1e37 / ((T + int(has_sink)) * (2 * bound + 1) ** n))
-        low = var._replace(shift=False, inv_stat=True, bounded_scores=True)
-        high = var._replace(shift=True, inv_stat=False, fast_rho=False, bounded_scores=False,
-                            head_resident=False, precise_output=True)
-        plan = _Plan(low, high, scale, bound, vmax, has_sink)
-    else:
-        plan = _Plan(var, None, scale, 0.0, 0.0, has_sink)
-    return _FlashFn.apply(q.contiguous(), k.contiguous(), v.contiguous(), sink, plan)
+        sink_logit = (torch.broadcast_to(sink_in.reshape(-1), (H,)) / unit).contiguous()
+        unit = 1.0
+    return _native.ops().flash(q, k, v, sink_logit, unit, plan)

@@ -13,54 +13,7 @@ from typing import Optional
 
 import torch
 
-from .. import _lib
-
-
-class _PrologueFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, qkv, q_gain, k_gain, cos, sin, H, eps):
-        B, T, three_d = qkv.shape
-        d = three_d // 3
-        D = d // H
-        dt = _lib.dtype_code(qkv.dtype)
-        out = torch.empty((3, B, H, T, D), dtype=qkv.dtype, device=qkv.device)
-        base = qkv.data_ptr()
-        esz = qkv.element_size()
-        _lib.call("algx_qk_prologue_fwd", _lib.c_ptr(base), _lib.c_ptr(base + d * esz),
-                  _lib.c_ptr(base + 2 * d * esz), three_d, _lib.ptr(q_gain), _lib.ptr(k_gain),
-                  _lib.ptr(cos), _lib.ptr(sin), _lib.ptr(out[0]), _lib.ptr(out[1]),
-                  _lib.ptr(out[2]), B, T, H, D, dt, float(eps), _lib.stream())
-        ctx.H, ctx.eps = H, eps
-        ctx.save_for_backward(qkv, q_gain, k_gain, cos, sin)
-        return out[0], out[1], out[2]
-
-    @staticmethod
-    def backward(ctx, dq_out, dk_out, dv_out):
-        qkv, q_gain, k_gain, cos, sin = ctx.saved_tensors
-        B, T, three_d = qkv.shape
-        d = three_d // 3
-        H = ctx.H
-        D = d // H
-        dt = _lib.dtype_code(qkv.dtype)
-        grads = [torch.zeros((B, H, T, D), dtype=qkv.dtype, device=qkv.device) if g is None
-                 else g.to(qkv.dtype).contiguous() for g in (dq_out, dk_out, dv_out)]
-        dqkv = torch.empty_like(qkv)
-        dqg = dkg = ws = None
-        if q_gain is not None:
-            dqg = torch.empty(D, dtype=torch.float32, device=qkv.device)
-            dkg = torch.empty(D, dtype=torch.float32, device=qkv.device)
-            ws = torch.empty(max(1, _lib.query("algx_qk_prologue_bwd_workspace_bytes", B, T, H, D,
-                                               dt)), dtype=torch.uint8, device=qkv.device)
-        base = dqkv.data_ptr()
-        esz = dqkv.element_size()
-        qb = qkv.data_ptr()
-        _lib.call("algx_qk_prologue_bwd", _lib.c_ptr(qb), _lib.c_ptr(qb + d * esz),
-                  _lib.ptr(q_gain), _lib.ptr(k_gain), _lib.ptr(cos), _lib.ptr(sin),
-                  _lib.ptr(grads[0]), _lib.ptr(grads[1]), _lib.ptr(grads[2]), _lib.c_ptr(base),
-                  _lib.c_ptr(base + d * esz), _lib.c_ptr(base + 2 * d * esz), three_d,
-                  _lib.ptr(dqg), _lib.ptr(dkg), _lib.ptr(ws), B, T, H, D, dt, float(ctx.eps),
-                  _lib.stream())
-        return dqkv, dqg, dkg, None, None, None, None
+from .. import _native
 
 
 def attention_prologue(qkv: torch.Tensor, n_heads: int, q_gain: Optional[torch.Tensor],
@@ -78,9 +31,7 @@ def attention_prologue(qkv: torch.Tensor, n_heads: int, q_gain: Optional[torch.T
     if (q_gain is None) != (k_gain is None) or (cos is None) != (sin is None):
         raise ValueError("gains and tables come in pairs")
     T = qkv.shape[1]
-    g32 = [None if g is None else g.to(torch.float32).contiguous() for g in (q_gain, k_gain)]
     tabs = [None if t is None else t[:T].to(torch.float32).contiguous() for t in (cos, sin)]
     if tabs[0] is not None and tuple(tabs[0].shape) != (T, 32):
         raise ValueError("rotation tables must be (T, 32)")
-    return _PrologueFn.apply(qkv.contiguous(), g32[0], g32[1], tabs[0], tabs[1], int(n_heads),
-                             float(eps))
+    return _native.ops().prologue(qkv, q_gain, k_gain, tabs[0], tabs[1], int(n_heads), float(eps))

@@ -13,64 +13,7 @@ return.
 
 import torch
 
-from .. import _lib
-
-
-class _NormFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, gain, eps):
-        rows = x.numel() // 64
-        y = torch.empty_like(x)
-        _lib.call("algx_qknorm_fwd", _lib.ptr(x), _lib.ptr(gain), _lib.ptr(y), rows, 64,
-                  _lib.dtype_code(x.dtype), float(eps), _lib.stream())
-        ctx.eps = eps
-        ctx.save_for_backward(x, gain)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, gain = ctx.saved_tensors
-        rows = x.numel() // 64
-        dt = _lib.dtype_code(x.dtype)
-        dy = dy.to(x.dtype).contiguous()
-        dx = torch.empty_like(x)
-        dgain = torch.empty(64, dtype=torch.float32, device=x.device)
-        ws = torch.empty(max(1, _lib.query("algx_qknorm_bwd_workspace_bytes", rows, 64, dt)),
-                         dtype=torch.uint8, device=x.device)
-        _lib.call("algx_qknorm_bwd", _lib.ptr(x), _lib.ptr(gain), _lib.ptr(dy), _lib.ptr(dx),
-                  _lib.ptr(dgain), _lib.ptr(ws), rows, 64, dt, float(ctx.eps), _lib.stream())
-        return dx, dgain.to(gain.dtype), None
-
-
-class _PairFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, gain_q, gain_k, eps):
-        rows = q.numel() // 64
-        yq, yk = torch.empty_like(q), torch.empty_like(k)
-        _lib.call("algx_qknorm_pair_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(gain_q),
-                  _lib.ptr(gain_k), _lib.ptr(yq), _lib.ptr(yk), rows, 64,
-                  _lib.dtype_code(q.dtype), float(eps), _lib.stream())
-        ctx.eps = eps
-        ctx.save_for_backward(q, k, gain_q, gain_k)
-        return yq, yk
-
-    @staticmethod
-    def backward(ctx, dyq, dyk):
-        q, k, gain_q, gain_k = ctx.saved_tensors
-        rows = q.numel() // 64
-        dt = _lib.dtype_code(q.dtype)
-        dyq = (torch.zeros_like(q) if dyq is None else dyq).to(q.dtype).contiguous()
-        dyk = (torch.zeros_like(k) if dyk is None else dyk).to(k.dtype).contiguous()
-        dxq, dxk = torch.empty_like(q), torch.empty_like(k)
-        dgq = torch.empty(64, dtype=torch.float32, device=q.device)
-        dgk = torch.empty(64, dtype=torch.float32, device=q.device)
-        ws = torch.empty(max(1, _lib.query("algx_qknorm_pair_bwd_workspace_bytes", rows, 64, dt)),
-                         dtype=torch.uint8, device=q.device)
-        _lib.call("algx_qknorm_pair_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(gain_q),
-                  _lib.ptr(gain_k), _lib.ptr(dyq), _lib.ptr(dyk), _lib.ptr(dxq), _lib.ptr(dxk),
-                  _lib.ptr(dgq), _lib.ptr(dgk), _lib.ptr(ws), rows, 64, dt, float(ctx.eps),
-                  _lib.stream())
-        return dxq, dxk, dgq.to(gain_q.dtype), dgk.to(gain_k.dtype), None
+from .. import _native
 
 
 def _check(x, gain, eps, block):
@@ -87,7 +30,7 @@ def _check(x, gain, eps, block):
 def qk_rms_norm(x, gain, eps=1e-5, *, block=1024):
     """RMS-normalize D=64 rows with a learned float32 gain (qk_norm.py:62-76)."""
     _check(x, gain, eps, block)
-    return _NormFn.apply(x.contiguous(), gain.contiguous(), float(eps))
+    return _native.ops().qk_norm(x, gain, float(eps))
 
 
 def qk_rms_norm_pair(q, k, gain_q, gain_k, eps=1e-5, *, block=1024):
@@ -99,5 +42,4 @@ def qk_rms_norm_pair(q, k, gain_q, gain_k, eps=1e-5, *, block=1024):
     _check(k, gain_k, eps, block)
     if q.shape != k.shape or q.dtype != k.dtype:
         raise ValueError("QK RMS pair needs q and k of one shape and dtype")
-    return _PairFn.apply(q.contiguous(), k.contiguous(), gain_q.contiguous(),
-                         gain_k.contiguous(), float(eps))
+    return _native.ops().qk_norm_pair(q, k, gain_q, gain_k, float(eps))

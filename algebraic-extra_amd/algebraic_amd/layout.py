@@ -32,34 +32,12 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 
 def _contig16(t: torch.Tensor) -> torch.Tensor:
     t = t.contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
-def _swap(x: torch.Tensor, B: int, P: int, Q: int, row: int) -> torch.Tensor:
-    """(B, P, Q, row) -> (B, Q, P, row) as a new tensor of x's dtype."""
-    x = _contig16(x)
-    out = torch.empty((B, Q, P, row), dtype=x.dtype, device=x.device)
-    _lib.call("algx_swap_axes", _lib.ptr(x), _lib.ptr(out), B, P, Q, row * x.element_size(),
-              _lib.stream())
-    return out
-
-
-class _HeadsToTokens(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, a):
-        B, H, T, D = a.shape
-        ctx.shape = (B, H, T, D)
-        return _swap(a, B, H, T, D).view(B, T, H * D)
-
-    @staticmethod
-    def backward(ctx, g):
-        B, H, T, D = ctx.shape
-        return _swap(g, B, T, H, D)
 
 
 def heads_to_tokens(a: torch.Tensor) -> torch.Tensor:
@@ -68,7 +46,7 @@ def heads_to_tokens(a: torch.Tensor) -> torch.Tensor:
         raise ValueError("heads_to_tokens expects (B, H, T, D)")
     if (a.shape[-1] * a.element_size()) % 16:
         raise ValueError("heads_to_tokens: a row of D values must span a multiple of 16 bytes")
-    return _HeadsToTokens.apply(a)
+    return _native.ops().heads_to_tokens(a)
 
 
 def _transpose(x: torch.Tensor) -> torch.Tensor:
@@ -162,33 +140,7 @@ def weight_grad(x2: torch.Tensor, g2: torch.Tensor) -> torch.Tensor:
     """x2^T g2 in bf16 for x2 (T, din), g2 (T, dout) bf16: float32 sums of
     split-K chunks added in chunk order (algx_gemm_bf16_splitk)."""
     T, din = x2.shape
-    dout = g2.shape[1]
-    x2, g2 = _contig16(x2), _contig16(g2)
-    splits = splitk_splits(din, dout, T)
-    ws = torch.empty(_lib.query("algx_gemm_bf16_splitk_workspace_bytes", din, dout, splits),
-                     dtype=torch.uint8, device=x2.device)
-    out = torch.empty((din, dout), dtype=torch.bfloat16, device=x2.device)
-    _lib.call("algx_gemm_bf16_splitk", _lib.ptr(x2), _lib.ptr(g2), _lib.ptr(out), _lib.ptr(ws),
-              din, dout, T, 0, 0, din, dout, dout, splits, _lib.stream())
-    return out
-
-
-class _Project(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, w):
-        ctx.save_for_backward(x, w)
-        return x @ w
-
-    @staticmethod
-    def backward(ctx, g):
-        x, w = ctx.saved_tensors
-        din, dout = w.shape
-        g = g.contiguous()
-        dx = g @ w.t() if ctx.needs_input_grad[0] else None
-        dw = None
-        if ctx.needs_input_grad[1]:
-            dw = weight_grad(x.reshape(-1, din), g.reshape(-1, dout))
-        return dx, dw
+    return _native.ops().weight_grad(x2, g2, splitk_splits(din, g2.shape[1], T))
 
 
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -200,5 +152,5 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if (x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda
             or din % 8 or dout % 8 or T % 32 or T == 0):
         return x @ w
-    return _Project.apply(x, w)
+    return _native.ops().project(x, w, splitk_splits(din, dout, T))
 

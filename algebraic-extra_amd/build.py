@@ -1,25 +1,30 @@
-"""Build libalgx.so (gfx950) in-tree with hipcc.
+"""Build libalgx.so (gfx950) and the torch operators over it in-tree.
 
     python algebraic-extra_amd/build.py            # compile every csrc/*.hip, link
     python algebraic-extra_amd/build.py --asm      # also write gfx950 ISA to _build/
 
 Each translation unit is compiled separately (in parallel) and linked into
-``algebraic_amd/libalgx.so`` next to the Python package that loads it.
+``algebraic_amd/libalgx.so`` next to the Python package that loads it;
+``csrc/torch_ops.cpp`` is compiled against the installed torch's headers to the
+extension module ``algebraic_amd/_ops.so``, which links that library.
 """
 
 import argparse
 import concurrent.futures as cf
 import glob
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 OUT = os.path.join(HERE, "algebraic_amd", "libalgx.so")
+OPS = os.path.join(HERE, "algebraic_amd", "_ops.so")
 ARCH = "gfx950"
 # Extra flags per translation unit: the MFMA kernels keep their accumulators in
 # architectural VGPRs so the VALU reads them without accvgpr copies.
@@ -65,18 +70,49 @@ def _compile(src, asm):
     return obj
 
 
+def _compile_ops():
+    torch = os.path.dirname(importlib.util.find_spec("torch").origin)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    obj = os.path.join(BUILD, "torch_ops.o")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_ops", "-I", os.path.join(ROOT, "include"),
+           "-isystem", os.path.join(torch, "include"),
+           "-isystem", os.path.join(torch, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"),
+           "-isystem", sysconfig.get_paths()["include"],
+           "-c", os.path.join(CSRC, "torch_ops.cpp"), "-o", obj]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compile failed: torch_ops.cpp\n{res.stderr}")
+    return obj, os.path.join(torch, "lib")
+
+
+def _link_ops(obj, torch_lib):
+    tmp = OPS + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", tmp, obj, "-L", os.path.dirname(OUT),
+           "-l:libalgx.so", "-L", torch_lib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link failed: _ops.so\n{res.stderr}")
+    os.replace(tmp, OPS)
+
+
 def build(asm=False, jobs=None):
     os.makedirs(BUILD, exist_ok=True)
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    jobs = jobs or min(8, len(sources), os.cpu_count() or 1)
+    jobs = jobs or min(8, len(sources) + 1, os.cpu_count() or 1)
     with cf.ThreadPoolExecutor(jobs) as ex:
+        ops = ex.submit(_compile_ops)
         objs = list(ex.map(lambda s: _compile(s, asm), sources))
+        ops_obj, torch_lib = ops.result()
     tmp = OUT + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-o", tmp] + objs
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed\n{res.stderr}")
     os.replace(tmp, OUT)
+    _link_ops(ops_obj, torch_lib)
     return OUT
 
 
