@@ -18,15 +18,13 @@ compute-dtype copies of the stacked weights for its fused projections.
 (din, dout)). Forward and input gradient are plain library GEMMs (hipBLASLt
 through torch); the weight gradient ``x^T dY``, whose K is the batch's token
 count while din x dout is one weight, runs on libalgx's split-K GEMM
-(algx_gemm_bf16_splitk): the library's choice for these shapes leaves most
+(algx_weight_grad): the library's choice for these shapes leaves most
 of the GPU idle (16 to 84 output tiles of 256 x 256 over 256 compute units).
 
 The first two accept any dtype whose rows (heads_to_tokens: D elements) span a
 multiple of 16 bytes (transpose_last2: 2- or 4-byte elements); all return new
 contiguous tensors.
 """
-
-import math
 
 import ctypes
 
@@ -125,22 +123,10 @@ def concat_cast(parts, dtype: torch.dtype) -> torch.Tensor:
 __all__ = ["heads_to_tokens", "transpose_last2", "concat_cast"]
 
 
-def splitk_splits(M: int, N: int, K: int) -> int:
-    """Chunks of K for algx_gemm_bf16_splitk: the fewest (a power of two)
-    whose workgroups cover 160 of the 256 compute units, keeping chunks of
-    at least 256 rows that are whole 32-row stages."""
-    tiles = math.ceil(M / 256) * math.ceil(N / 256)
-    s = 1
-    while tiles * s < 160 and K % (64 * s) == 0 and K // (2 * s) >= 256:
-        s *= 2
-    return s
-
-
 def weight_grad(x2: torch.Tensor, g2: torch.Tensor) -> torch.Tensor:
     """x2^T g2 in bf16 for x2 (T, din), g2 (T, dout) bf16: float32 sums of
-    split-K chunks added in chunk order (algx_gemm_bf16_splitk)."""
-    T, din = x2.shape
-    return _native.ops().weight_grad(x2, g2, splitk_splits(din, g2.shape[1], T))
+    chunks of T added in chunk order (algx_weight_grad)."""
+    return _native.ops().weight_grad(x2, g2)
 
 
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -152,5 +138,5 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if (x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda
             or din % 8 or dout % 8 or T % 32 or T == 0):
         return x @ w
-    return _native.ops().project(x, w, splitk_splits(din, dout, T))
+    return _native.ops().project(x, w)
 

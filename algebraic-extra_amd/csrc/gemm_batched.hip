@@ -194,7 +194,7 @@ BatchFn pick_batched(bool akc, bool bkc, bool dma, bool sym) {
 
 // Split-K product (the weight gradients of the model's projections, K = the
 // token count): C[m][n] = cast(sum_k opA(m, k) opB(n, k)) with K cut into
-// `splits` chunks of Kc. Workgroup b forms chunk b / ntiles of tile
+// `splits` chunks of Kc (the last may be shorter). Workgroup b forms chunk b / ntiles of tile
 // b % ntiles (256 x 256, m along the core's M axis, so a lane's sixteen
 // accumulators are sixteen rows of one column and each store instruction
 // covers 32 consecutive columns of two rows) and stores it in float32 to the
@@ -205,7 +205,7 @@ struct SplitK {
   const bf16* B;
   float* P;  // workspace: splits x M x N float32
   int64_t lda, ldb;
-  int M, N, Kc, splits, tiles_n;
+  int M, N, K, Kc, splits, tiles_m, tiles_n;
 };
 
 template <bool AKC, bool BKC, bool DMA>
@@ -213,15 +213,30 @@ __global__ __launch_bounds__(kThreads) void splitk_gemm_kernel(SplitK p) {
   GEMM_LDS_STAGES;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 5, c32 = lane & 31;
   const int wm = w / NWN, wn = w % NWN;
-  const int ntiles = (int)gridDim.x / p.splits;
-  const int split = (int)blockIdx.x / ntiles, tile = (int)blockIdx.x % ntiles;
-  const int m0 = (tile / p.tiles_n) * BM, n0 = (tile % p.tiles_n) * BN;
+  // Workgroups are dealt to the 8 XCDs round-robin by index. From 192 units on
+  // each XCD takes a run of consecutive ones (chunk-major, the shorter side of
+  // the tile grid fastest), so that the workgroups running on it at a time
+  // read a few rows of tiles of each operand through its L2 at about the same
+  // k: 768 x 2304 over 16384 tokens 79 -> 68 us, 1024 x 5376 189 -> 176. With
+  // fewer, operand traffic is no bound and the same lines asked for at once
+  // cost more: 384 x 2048 over 4096 tokens (128 units) 19.3 us in runs, 15.8
+  // in plain order.
+  const int ntiles = p.tiles_m * p.tiles_n, per_xcd = (int)gridDim.x / 8;
+  const bool runs = ntiles * p.splits >= 192;
+  const int unit =
+      runs ? ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+  if (unit >= ntiles * p.splits) return;
+  const int split = unit / ntiles, tile = unit % ntiles;
+  const bool m_fast = p.tiles_m <= p.tiles_n;
+  const int m0 = (m_fast ? tile % p.tiles_m : tile / p.tiles_n) * BM;
+  const int n0 = (m_fast ? tile / p.tiles_m : tile % p.tiles_n) * BN;
   const int64_t k0 = (int64_t)split * p.Kc;
-  const Operand Aop{p.A + (AKC ? k0 : k0 * p.lda), p.lda, p.M, p.Kc};
-  const Operand Bop{p.B + (BKC ? k0 : k0 * p.ldb), p.ldb, p.N, p.Kc};
+  const int kc = (int)min((int64_t)p.Kc, p.K - k0);
+  const Operand Aop{p.A + (AKC ? k0 : k0 * p.lda), p.lda, p.M, kc};
+  const Operand Bop{p.B + (BKC ? k0 : k0 * p.ldb), p.ldb, p.N, kc};
   Acc acc;
   if constexpr (DMA)
-    gemm_tile_dma<AKC, BKC>(Aop, Bop, m0, n0, ring, acc, tid);
+    gemm_tile_range<AKC, BKC>(Aop, Bop, m0, n0, 0, (kc + BK - 1) / BK, ring, acc, tid);
   else
     gemm_tile<AKC, BKC>(Aop, Bop, m0, n0, s0, s0 + 2 * kStageElems, acc, tid);
   // acc.v[i][j][r] = partial C[m0 + WTM wm + 32 i + 8 (r / 4) + 4 g + r % 4][n0 + WTN wn + 32 j + c32]
@@ -265,6 +280,58 @@ template <bool DMA> SplitFn pick_splitk_as(bool akc, bool bkc) {
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// The product and the sum of its slices; K in `splits` chunks of Kc.
+int32_t launch_splitk(const void* A, const void* B, void* C, void* workspace, int M, int N, int K,
+                      int Kc, bool a_kc, bool b_kc, int64_t lda, int64_t ldb, int64_t ldc,
+                      int splits, hipStream_t s) {
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int64_t grid = ((int64_t)tiles_m * tiles_n * splits + 7) / 8 * 8;
+  if (grid > 0x7fffffff) return fail("gemm_bf16_splitk: too many tiles");
+  const SplitK p{(const bf16*)A, (const bf16*)B, (float*)workspace, lda, ldb, M, N, K, Kc, splits,
+                 tiles_m, tiles_n};
+  // [k][mn] operands may end inside a 32-wide stage, k-contiguous ones not.
+  const bool dma = (Kc % BK == 0 || splits == 1) && ((!a_kc && !b_kc) || K % BK == 0) &&
+                   dma_span_ok(Operand{nullptr, lda, M, Kc}, a_kc) &&
+                   dma_span_ok(Operand{nullptr, ldb, N, Kc}, b_kc);
+  SplitFn fn = dma ? pick_splitk_as<true>(a_kc, b_kc) : pick_splitk_as<false>(a_kc, b_kc);
+  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(kThreads), 0, s, p);
+  if (int32_t rc = check_launch("gemm_bf16_splitk")) return rc;
+  int64_t nb = ((int64_t)M * N / 4 + 255) / 256;
+  if (nb > 4096) nb = 4096;
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)nb), dim3(256), 0, s,
+                     (const float*)workspace, (bf16*)C, M, N, (int64_t)ldc, splits);
+  return check_launch("gemm_bf16_splitk_reduce");
+}
+
+// Chunks of a weight gradient's K = tokens. One round of workgroups over the
+// 256 compute units is the aim, and its fullness counts: with powers of two
+// only, the 350M model's gradients filled 168 to 192 of them. The cost of s
+// chunks, in 32-row stages: the rounds, each with a chunk's stages and about 20
+// stages' worth of filling the ring and storing the slice, and the slices
+// written and read again at about 10 TB/s (a stage is about 0.55 us; the slices
+// mostly stay in the Infinity Cache). Chunks of at least 8 stages. Over 16384
+// tokens, with the order above: 1024 x 5376 in 3 chunks (252 workgroups)
+// instead of 2 (168) 205 -> 176 us, 1024 x 3072 in 5 instead of 4 136 -> 120-125,
+// 2688 x 1024 in 5 instead of 4 105 -> 96, 768 x 768 57 -> 38.
+int wgrad_splits(int M, int N, int K) {
+  constexpr int kUnits = 256;
+  const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  const int stages = (K + BK - 1) / BK;
+  const double slice = (double)M * N * 8 / 10e12 / 0.55e-6;
+  int best = 1;
+  double least = 0.0;
+  for (int s = 1; s <= 64 && (s == 1 || stages / s >= 8); ++s) {
+    const int per = (stages + s - 1) / s;
+    if ((stages + per - 1) / per != s) continue;  // the same chunks as fewer splits
+    const double cost = (double)((tiles * s + kUnits - 1) / kUnits) * (per + 20) + slice * s;
+    if (s == 1 || cost < least) {
+      least = cost;
+      best = s;
+    }
+  }
+  return best;
+}
 
 // Checks one batch's arguments and fills its descriptor (tile counts are set
 // by the launch, which knows whether the symmetric schedule runs).
@@ -407,23 +474,29 @@ extern "C" int32_t algx_gemm_bf16_splitk(const void* A, const void* B, void* C, 
     return fail("gemm_bf16_splitk: operands must be 16-byte aligned");
   if (lda < (a_kc ? K : M) || ldb < (b_kc ? K : N) || ldc < N)
     return fail("gemm_bf16_splitk: leading dimension below the row length");
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int64_t grid = (int64_t)tiles_m * tiles_n * splits;
-  if (grid > 0x7fffffff) return fail("gemm_bf16_splitk: too many tiles");
-  hipStream_t s = (hipStream_t)stream;
-  const SplitK p{(const bf16*)A, (const bf16*)B, (float*)workspace, lda, ldb, M, N, Kc, splits,
-                 tiles_n};
-  const bool dma = Kc % BK == 0 && dma_span_ok(Operand{nullptr, lda, M, Kc}, a_kc != 0) &&
-                   dma_span_ok(Operand{nullptr, ldb, N, Kc}, b_kc != 0);
-  SplitFn fn = dma ? pick_splitk_as<true>(a_kc != 0, b_kc != 0)
-                   : pick_splitk_as<false>(a_kc != 0, b_kc != 0);
-  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(kThreads), 0, s, p);
-  if (int32_t rc = check_launch("gemm_bf16_splitk")) return rc;
-  int64_t nb = ((int64_t)M * N / 4 + 255) / 256;
-  if (nb > 4096) nb = 4096;
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)nb), dim3(256), 0, s,
-                     (const float*)workspace, (bf16*)C, M, N, (int64_t)ldc, splits);
-  return check_launch("gemm_bf16_splitk_reduce");
+  return launch_splitk(A, B, C, workspace, M, N, K, Kc, a_kc != 0, b_kc != 0, lda, ldb, ldc,
+                       splits, (hipStream_t)stream);
+}
+
+extern "C" int64_t algx_weight_grad_workspace_bytes(int32_t T, int32_t din, int32_t dout) {
+  if (T <= 0 || din <= 0 || dout <= 0) return 0;
+  return (int64_t)wgrad_splits(din, dout, T) * din * dout * (int64_t)sizeof(float);
+}
+
+extern "C" int32_t algx_weight_grad(const void* x, const void* g, void* dw, void* workspace,
+                                    int32_t T, int32_t din, int32_t dout, void* stream) {
+  if (T < 0 || din < 0 || dout < 0) return fail("weight_grad: negative size");
+  if (din == 0 || dout == 0) return 0;
+  if (T == 0) return fail("weight_grad: no tokens");
+  if (x == nullptr || g == nullptr || dw == nullptr || workspace == nullptr)
+    return fail("weight_grad: null pointer");
+  if (din % 8 || dout % 8) return fail("weight_grad: widths must be multiples of 8");
+  if (!aligned16(x) || !aligned16(g) || !aligned16(dw) || !aligned16(workspace))
+    return fail("weight_grad: operands must be 16-byte aligned");
+  const int stages = (T + BK - 1) / BK, want = wgrad_splits(din, dout, T);
+  const int per = (stages + want - 1) / want;
+  return launch_splitk(x, g, dw, workspace, din, dout, T, per * BK, false, false, din, dout, dout,
+                       want, (hipStream_t)stream);
 }
 
 extern "C" int32_t algx_gemm_bf16_grouped(const algx_gemm_batch* groups, int32_t ngroups,

@@ -513,23 +513,21 @@ Tensor heads_to_tokens(const Tensor& a) {
   return HeadsToTokens::apply(a);
 }
 
-// x2^T g2 in bf16 for x2 (T, din), g2 (T, dout): float32 sums of split-K chunks
-// added in chunk order.
-Tensor weight_grad(const Tensor& x, const Tensor& g, int64_t splits) {
+// x^T g in bf16 for x (T, din), g (T, dout): float32 sums of chunks of T added
+// in chunk order.
+Tensor weight_grad(const Tensor& x, const Tensor& g) {
   const Tensor x2 = aligned(x), g2 = aligned(g);
   const int64_t T = x2.size(0), din = x2.size(1), dout = g2.size(1);
-  Tensor ws = scratch(algx_gemm_bf16_splitk_workspace_bytes(din, dout, splits), x2);
+  Tensor ws = scratch(algx_weight_grad_workspace_bytes(T, din, dout), x2);
   Tensor out = at::empty({din, dout}, x2.options());
-  check(algx_gemm_bf16_splitk(ptr(x2), ptr(g2), ptr(out), ptr(ws), din, dout, T, 0, 0, din, dout,
-                              dout, splits, stream()),
-        "algx_gemm_bf16_splitk");
+  check(algx_weight_grad(ptr(x2), ptr(g2), ptr(out), ptr(ws), T, din, dout, stream()),
+        "algx_weight_grad");
   return out;
 }
 
 struct Project : Function<Project> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, int64_t splits) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
     ctx->save_for_backward({x, w});
-    ctx->saved_data["splits"] = splits;
     return at::matmul(x, w);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -540,15 +538,12 @@ struct Project : Function<Project> {
     Tensor dx, dw;
     if (ctx->needs_input_grad(0)) dx = at::matmul(g, w.t());
     if (ctx->needs_input_grad(1))
-      dw = weight_grad(x.reshape({-1, din}), g.reshape({-1, dout}),
-                       ctx->saved_data["splits"].toInt());
-    return {dx, dw, Tensor()};
+      dw = weight_grad(x.reshape({-1, din}), g.reshape({-1, dout}));
+    return {dx, dw};
   }
 };
 
-Tensor project(const Tensor& x, const Tensor& w, int64_t splits) {
-  return Project::apply(x, w, splits);
-}
+Tensor project(const Tensor& x, const Tensor& w) { return Project::apply(x, w); }
 
 }  // namespace
 

@@ -385,6 +385,13 @@ int64_t algx_gemm_bf16_splitk_workspace_bytes(int32_t M, int32_t N, int32_t spli
 int32_t algx_gemm_bf16_splitk(const void* A, const void* B, void* C, void* workspace, int32_t M,
                               int32_t N, int32_t K, int32_t a_kc, int32_t b_kc, int64_t lda,
                               int64_t ldb, int64_t ldc, int32_t splits, void* stream);
+/* algx_weight_grad: the same for one projection, dw (din, dout) = x^T g of
+ * bf16 x (T, din) and g (T, dout), the chunks of T chosen here (the last one
+ * may be shorter; any T > 0). din and dout multiples of 8, pointers 16-byte
+ * aligned. */
+int64_t algx_weight_grad_workspace_bytes(int32_t T, int32_t din, int32_t dout);
+int32_t algx_weight_grad(const void* x, const void* g, void* dw, void* workspace, int32_t T,
+                         int32_t din, int32_t dout, void* stream);
 /* algx_gemm_bf16_grouped: up to 4 batches of algx_gemm_bf16_batched products
  * in one launch (the operands, sizes and strides of each group its own; the
  * operand layouts, symmetry and alpha/beta shared). Muon orthogonalises

@@ -276,3 +276,28 @@ def test_operands_beyond_32bit_lane_offsets_take_the_staged_path():
     _check(C2, want)
     del big
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("T,din,dout", [(1, 8, 8), (31, 264, 40), (33, 256, 512), (1000, 384, 1152),
+                                        (2055, 1032, 520), (8192, 768, 2304), (4096, 1024, 5376)])
+def test_weight_grad_any_token_count(T, din, dout):
+    """algx_weight_grad: token counts that end inside a 32-row stage or a
+    chunk, one chunk and many, fewer units than XCD runs take and more, into
+    outputs and a workspace that start as NaN; two calls agree bit for bit."""
+    from algebraic_amd import _lib
+    g = torch.Generator(device=DEV).manual_seed(T + din + dout)
+    x = torch.randn((T, din), generator=g, device=DEV).bfloat16()
+    dy = torch.randn((T, dout), generator=g, device=DEV).bfloat16()
+    outs = []
+    for _ in range(2):
+        C = torch.full((din, dout), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ws = torch.full((_lib.query("algx_weight_grad_workspace_bytes", T, din, dout) // 4,),
+                        float("nan"), device=DEV)
+        _lib.call("algx_weight_grad", _lib.ptr(x), _lib.ptr(dy), _lib.ptr(C), _lib.ptr(ws), T, din,
+                  dout, _lib.stream())
+        outs.append(C)
+    want = x.double().t() @ dy.double()
+    # one bf16 rounding of float32 sums of exact bf16 products
+    bound = 2 ** -8 * want.abs() + 5e-5 * (x.double().abs().t() @ dy.double().abs())
+    assert ((outs[0].double() - want).abs() <= bound).all()
+    assert torch.equal(outs[0], outs[1])
