@@ -60,6 +60,10 @@ SIGNATURES = {
     "algx_attn_forward_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
     "algx_attn_forward": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32,
                                  _i32, _i32, _f32, _f32, _f32, _VP, _VP, _p]),
+    "algx_attn_forward_unit": (_i32, [_p, _p, _p, _p, _f32, _p, _p, _p, _p, _p, _p, _p, _i32, _i32,
+                                      _i32, _i32, _i32, _f32, _f32, _f32, _VP, _VP, _p]),
+    "algx_attn_bwd_unit": (_i32, [_p, _p, _p, _p, _f32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i32,
+                                  _i32, _i32, _i32, _i32, _i32, _f32, _VP, _VP, _p, _p]),
     "algx_attn_forward_noalloc": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i32, _i32,
                                          _i32, _i32, _i32, _f32, _f32, _f32, _VP, _VP, _p]),
     "algx_attn_bwd_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),

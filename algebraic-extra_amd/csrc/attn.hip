@@ -122,7 +122,7 @@ extern "C" int32_t algx_attn_prepare(const void* q, const void* k, const void* v
   if (guard != nullptr && (k == nullptr || v == nullptr))
     return fail("attn_prepare: the guard needs k and v");
   if (int32_t rc = check_aligned("attn_prepare", {q, k, v, q_s})) return rc;
-  return launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound, vmax,
+  return launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound, vmax, 1.0f,
                         (hipStream_t)stream);
 }
 
@@ -164,13 +164,14 @@ extern "C" int64_t algx_attn_forward_workspace_bytes(int32_t B, int32_t H, int32
   return fwd_fused_partials(B, H, T) * 3 * (int64_t)sizeof(float);
 }
 
-extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v,
-                                     const float* sink, void* q_s, void* o, float* o_precise,
-                                     float* stat, int32_t* guard, void* workspace,
-                                     void* bwd_workspace, int32_t B, int32_t H, int32_t T,
-                                     int32_t D, int32_t dtype, float q_scale, float bound,
-                                     float vmax, const algx_attn_variant* low,
-                                     const algx_attn_variant* high, void* stream) {
+extern "C" int32_t algx_attn_forward_unit(const void* q, const void* k, const void* v,
+                                          const float* sink, float sink_unit, void* q_s, void* o,
+                                          float* o_precise, float* stat, int32_t* guard,
+                                          void* workspace, void* bwd_workspace, int32_t B,
+                                          int32_t H, int32_t T, int32_t D, int32_t dtype,
+                                          float q_scale, float bound, float vmax,
+                                          const algx_attn_variant* low,
+                                          const algx_attn_variant* high, void* stream) {
   if (int32_t rc = check_shape(B, H, T, D, dtype)) return rc;
   KVariant kl{}, kh{};
   if (int32_t rc = to_kvar(low, kl, "low")) return rc;
@@ -179,6 +180,7 @@ extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v
   } else {
     kh = kl;
   }
+  kl.sink_unit = kh.sink_unit = sink_unit;
   if ((int64_t)B * H * T == 0) return 0;
   if (q == nullptr || k == nullptr || v == nullptr || q_s == nullptr || o == nullptr ||
       stat == nullptr)
@@ -203,7 +205,7 @@ extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v
   if (mfma && bwd_workspace != nullptr)
     if (int32_t rc = fill_f32((float*)bwd_workspace, acc_bytes(B, H, T, D) / 4, 0.0f, s)) return rc;
   if (int32_t rc = launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound,
-                                  vmax, s))
+                                  vmax, sink_unit, s))
     return rc;
   if (int32_t rc = launch_fwd_generic(q_s, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kl,
                                       guard, 1, s))
@@ -212,6 +214,18 @@ extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v
     return launch_fwd_generic(q_s, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kh, guard,
                               0, s);
   return 0;
+}
+
+extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v,
+                                     const float* sink, void* q_s, void* o, float* o_precise,
+                                     float* stat, int32_t* guard, void* workspace,
+                                     void* bwd_workspace, int32_t B, int32_t H, int32_t T,
+                                     int32_t D, int32_t dtype, float q_scale, float bound,
+                                     float vmax, const algx_attn_variant* low,
+                                     const algx_attn_variant* high, void* stream) {
+  return algx_attn_forward_unit(q, k, v, sink, 1.0f, q_s, o, o_precise, stat, guard, workspace,
+                                bwd_workspace, B, H, T, D, dtype, q_scale, bound, vmax, low, high,
+                                stream);
 }
 
 extern "C" int64_t algx_attn_bwd_workspace_bytes(int32_t B, int32_t H, int32_t T, int32_t D) {
@@ -223,13 +237,14 @@ extern "C" int64_t algx_attn_bwd_workspace_bytes(int32_t B, int32_t H, int32_t T
   return acc + di + shares;
 }
 
-extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, const float* sink,
-                                 const void* o, const float* o_precise, const float* stat,
-                                 const void* dout, void* dq, void* dk, void* dv, float* dsink,
-                                 void* workspace, int32_t workspace_state, int32_t B, int32_t H,
-                                 int32_t T, int32_t D, int32_t dtype, float q_scale,
-                                 const algx_attn_variant* low, const algx_attn_variant* high,
-                                 const int32_t* guard, void* stream) {
+extern "C" int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* v,
+                                      const float* sink, float sink_unit, const void* o,
+                                      const float* o_precise, const float* stat, const void* dout,
+                                      void* dq, void* dk, void* dv, float* dsink, void* workspace,
+                                      int32_t workspace_state, int32_t B, int32_t H, int32_t T,
+                                      int32_t D, int32_t dtype, float q_scale,
+                                      const algx_attn_variant* low, const algx_attn_variant* high,
+                                      const int32_t* guard, void* stream) {
   if (int32_t rc = check_shape(B, H, T, D, dtype)) return rc;
   KVariant kl{}, kh{};
   if (int32_t rc = to_kvar(low, kl, "low")) return rc;
@@ -238,6 +253,7 @@ extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, co
   } else {
     kh = kl;
   }
+  kl.sink_unit = kh.sink_unit = sink_unit;
   if (workspace_state != ALGX_ATTN_WS_RAW && workspace_state != ALGX_ATTN_WS_CLEARED)
     return fail("attn_bwd: workspace_state must be ALGX_ATTN_WS_RAW or ALGX_ATTN_WS_CLEARED");
   hipStream_t s = (hipStream_t)stream;
@@ -260,7 +276,8 @@ extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, co
   // accumulator unless the forward already did (a workspace it prepared).
   const bool cleared = mfma && workspace_state == ALGX_ATTN_WS_CLEARED;
   float* shares = (float*)((char*)di + ((rows * (int64_t)sizeof(float) + 255) / 256) * 256);
-  const SinkGrad sg{shares, sink != nullptr ? dsink : nullptr, pre_blocks(T, D, dtype), B, H};
+  const SinkGrad sg{shares, sink != nullptr ? dsink : nullptr, pre_blocks(T, D, dtype), B, H,
+                    sink_unit};
   if (int32_t rc = launch_bwd_pre(dout, o, o_precise, stat, sink, di,
                                   mfma && !cleared ? dq_acc : nullptr,
                                   sg.dsink != nullptr ? shares : nullptr, B, H, T, D, dtype, kl,
@@ -282,6 +299,18 @@ extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, co
     return launch_bwd_generic(q, k, v, stat, di, dout, dq, dk, dv, B, H, T, D, dtype, q_scale, kh,
                               guard, 0, s);
   return 0;
+}
+
+extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, const float* sink,
+                                 const void* o, const float* o_precise, const float* stat,
+                                 const void* dout, void* dq, void* dk, void* dv, float* dsink,
+                                 void* workspace, int32_t workspace_state, int32_t B, int32_t H,
+                                 int32_t T, int32_t D, int32_t dtype, float q_scale,
+                                 const algx_attn_variant* low, const algx_attn_variant* high,
+                                 const int32_t* guard, void* stream) {
+  return algx_attn_bwd_unit(q, k, v, sink, 1.0f, o, o_precise, stat, dout, dq, dk, dv, dsink,
+                            workspace, workspace_state, B, H, T, D, dtype, q_scale, low, high,
+                            guard, stream);
 }
 
 // algx_attn_forward with the guard partials in the library's per-device

@@ -9,16 +9,18 @@ int32_t guard_words();
 // q_s = cast(q * q_scale); with a guard buffer also the range-guard word.
 int32_t launch_prepare(const void* q, const void* k, const void* v, const float* sink, void* q_s,
                        int32_t* guard, int B, int H, int T, int D, int dtype, float q_scale,
-                       float bound, float vmax, hipStream_t s);
+                       float bound, float vmax, float sink_unit, hipStream_t s);
 // Guard word from `nblocks` triples of partial maxima (|q_s|^2, |k|^2, |v|).
 int32_t launch_guard_finish(const float* partial, int nblocks, const float* sink, int H,
-                            float bound, float vmax, int32_t* guard, hipStream_t s);
+                            float bound, float vmax, float sink_unit, int32_t* guard,
+                            hipStream_t s);
 // The sink gradient's shares of the backward pre-pass (nblk per (b, h)) and
 // where their sums go; dsink null: no sink gradient.
 struct SinkGrad {
   const float* part;
   float* dsink;
   int nblk, B, H;
+  float unit;  // the sink's
 };
 // Row pre-pass of the backward: di (and, with a sink and sink_part, each
 // block's share of the sink gradient, pre_blocks() per (b, h)), and the dQ

@@ -104,7 +104,8 @@ __global__ __launch_bounds__(256) void scale_kernel(const T* __restrict__ q, T* 
 __global__ __launch_bounds__(256) void guard_finish_kernel(const float* __restrict__ partial,
                                                            int nblocks, const float* sink, int H,
                                                            float bound_sq, float bound_s,
-                                                           float vmax, int32_t* guard) {
+                                                           float vmax, float sink_unit,
+                                                           int32_t* guard) {
   __shared__ float red[3][256];
   float mq = 0.0f, mk = 0.0f, mv = 0.0f;
   for (int b = threadIdx.x; b < nblocks; b += 256) {
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256) void guard_finish_kernel(const float* __restri
   if (threadIdx.x == 0) {
     float ms = 0.0f;
     if (sink != nullptr)
-      for (int h = 0; h < H; ++h) ms = __builtin_fmaxf(ms, nan_to_inf(__builtin_fabsf(sink[h])));
+      for (int h = 0; h < H; ++h) ms = __builtin_fmaxf(ms, nan_to_inf(__builtin_fabsf(sink[h] / sink_unit)));
     const float q2 = red[0][0], k2 = red[1][0], vm = red[2][0];
     bool ok = q2 * k2 <= bound_sq;
     if (sink != nullptr) ok = ok && ms <= bound_s;
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(
   const int bh = blockIdx.y, h = bh % H;
   const int64_t head = (int64_t)bh * T_;
   const bool has_sink = sink != nullptr;
-  const float b = has_sink ? sink[h] : 0.0f;
+  const float b = has_sink ? var.sink(sink, h) : 0.0f;
   float ds_acc = 0.0f;
   const int rows_per_iter = 4 * RPW;
   for (int t = blockIdx.x * rows_per_iter + (threadIdx.x >> 6) * RPW + rw; t < T_;
@@ -209,10 +210,10 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(
   }
 }
 
-// dsink[h] = the sum over the batch of head h's row-block shares (nblk per
+// dsink[h] = 1 / unit times the sum over the batch of head h's row-block shares (nblk per
 // (b, h)), by one block of 256 threads.
 __device__ __forceinline__ void sum_sink(const float* __restrict__ part, int nblk, int B, int H,
-                                         int h, float* __restrict__ dsink) {
+                                         int h, float unit, float* __restrict__ dsink) {
   float s = 0.0f;
   for (int i = threadIdx.x; i < B * nblk; i += 256)
     s += part[((int64_t)(i / nblk) * H + h) * nblk + i % nblk];
@@ -221,13 +222,13 @@ __device__ __forceinline__ void sum_sink(const float* __restrict__ part, int nbl
   __shared__ float red[4];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) dsink[h] = (red[0] + red[1]) + (red[2] + red[3]);
+  if (threadIdx.x == 0) dsink[h] = ((red[0] + red[1]) + (red[2] + red[3])) / unit;
 }
 
 __global__ __launch_bounds__(256) void sink_finish_kernel(const float* __restrict__ part, int nblk,
-                                                          int B, int H,
+                                                          int B, int H, float unit,
                                                           float* __restrict__ dsink) {
-  sum_sink(part, nblk, B, H, blockIdx.x, dsink);
+  sum_sink(part, nblk, B, H, blockIdx.x, unit, dsink);
 }
 
 // dq = cast(cast(acc * slope) * q_scale): the kernel's dQ output rounding
@@ -243,7 +244,7 @@ __global__ __launch_bounds__(256) void dq_finish_kernel(const float* __restrict_
                                                         float q_scale, SinkGrad sg) {
   const int nsink = sg.dsink != nullptr ? sg.H : 0;
   if ((int)blockIdx.x < nsink) {
-    sum_sink(sg.part, sg.nblk, sg.B, sg.H, blockIdx.x, sg.dsink);
+    sum_sink(sg.part, sg.nblk, sg.B, sg.H, blockIdx.x, sg.unit, sg.dsink);
     return;
   }
   const KVariant& var = guard_in_range(guard) ? low : high;
@@ -266,7 +267,7 @@ int32_t guard_words() { return 8 + 3 * kGuardBlocks; }
 
 int32_t launch_prepare(const void* q, const void* k, const void* v, const float* sink, void* q_s,
                        int32_t* guard, int B, int H, int T, int D, int dtype, float q_scale,
-                       float bound, float vmax, hipStream_t s) {
+                       float bound, float vmax, float sink_unit, hipStream_t s) {
   const int64_t rows = (int64_t)B * H * T;
   if (guard == nullptr) {
     const int64_t n = rows * D;
@@ -302,14 +303,15 @@ int32_t launch_prepare(const void* q, const void* k, const void* v, const float*
   }
 #undef GUARD_CASE
   if (int32_t rc = check_launch("attn_guard_partial")) return rc;
-  return launch_guard_finish(partial, (int)nb, sink, H, bound, vmax, guard, s);
+  return launch_guard_finish(partial, (int)nb, sink, H, bound, vmax, sink_unit, guard, s);
 }
 
 int32_t launch_guard_finish(const float* partial, int nblocks, const float* sink, int H,
-                            float bound, float vmax, int32_t* guard, hipStream_t s) {
+                            float bound, float vmax, float sink_unit, int32_t* guard,
+                            hipStream_t s) {
   const double b101 = (double)bound / 1.01;
   guard_finish_kernel<<<1, 256, 0, s>>>(partial, nblocks, sink, H, (float)(b101 * b101),
-                                        (float)b101, vmax, guard);
+                                        (float)b101, vmax, sink_unit, guard);
   return check_launch("attn_guard_finish");
 }
 
@@ -350,7 +352,7 @@ int32_t launch_bwd_pre(const void* dout, const void* o, const float* o_precise,
 }
 
 int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s) {
-  sink_finish_kernel<<<sg.H, 256, 0, s>>>(sg.part, sg.nblk, sg.B, sg.H, sg.dsink);
+  sink_finish_kernel<<<sg.H, 256, 0, s>>>(sg.part, sg.nblk, sg.B, sg.H, sg.unit, sg.dsink);
   return check_launch("attn_sink_finish");
 }
 

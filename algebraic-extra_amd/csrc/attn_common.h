@@ -18,6 +18,8 @@ struct KVariant {
   float clamp;
   float slope;   // n for asinh, 1 for softmax (flash.py:430, :441)
   int poly;      // bounded radical (radical.py:26-38)
+  float sink_unit = 1.0f;  // the sink array holds logits in units of this
+  __device__ __forceinline__ float sink(const float* p, int h) const { return p[h] / sink_unit; }
 };
 
 // rho and its slope factor r of the variant (flash.py:91-92).

@@ -126,7 +126,7 @@ __device__ __forceinline__ void fwd_body(
 
   const bool has_sink = sink != nullptr;
   float m_row, l_row;
-  sink_init(var, has_sink, has_sink ? sink[h] : 0.0f, m_row, l_row);
+  sink_init(var, has_sink, has_sink ? var.sink(sink, h) : 0.0f, m_row, l_row);
   if (g == 1) l_row = 0.0f;  // the two lane halves carry partial row sums
   f32x16 oacc[2];
   zero16(oacc[0]);
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void fwd_fallback_kernel(
   float ms = 0.0f;
   if (sink != nullptr)
     for (int h = 0; h < H; ++h) {
-      const float a = __builtin_fabsf(sink[h]);
+      const float a = __builtin_fabsf(hi.sink(sink, h));
       ms = __builtin_fmaxf(ms, a != a ? __builtin_inff() : a);
     }
   bool ok = tot[0] * tot[1] <= gin.bound_sq && tot[2] <= gin.vmax;

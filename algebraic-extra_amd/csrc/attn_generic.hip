@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kThreads) void fwd_generic_kernel(
   float m = noshift ? 0.0f : -__builtin_inff(), l = 0.0f;
   if (w == 0 && sink != nullptr) {
     float l0;
-    sink_init(var, true, sink[h], m, l0);
+    sink_init(var, true, var.sink(sink, h), m, l0);
     l = g == 0 ? l0 : 0.0f;
   }
   f32x4 acc[D / 16];

@@ -121,10 +121,7 @@ struct Flash : Function<Flash> {
                         bool need_grad) {
     const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3);
     Tensor guard, ws, bws, o_precise, s;
-    if (sink.has_value()) {
-      s = sink->reshape({-1});
-      s = unit == 1.0 ? s.contiguous() : s.div(unit);
-    }
+    if (sink.has_value()) s = sink->reshape({-1}).contiguous();
     if (plan->guarded) {
       guard = at::empty({algx_attn_guard_words()}, q.options().dtype(at::kInt));
       ws = scratch(algx_attn_forward_workspace_bytes(B, H, T, D), q);
@@ -132,10 +129,10 @@ struct Flash : Function<Flash> {
     Tensor q_s = at::empty_like(q), o = at::empty_like(q), stat = f32({B, H, T}, q);
     if (plan->precise()) o_precise = f32(q.sizes(), q);
     if (need_grad) bws = scratch(algx_attn_bwd_workspace_bytes(B, H, T, D), q);
-    check(algx_attn_forward(ptr(q), ptr(k), ptr(v), fptr(s), ptr(q_s), ptr(o), fptr(o_precise),
-                            fptr(stat), static_cast<int32_t*>(ptr(guard)), ptr(ws), ptr(bws), B, H,
-                            T, D, dtype_code(q), plan->scale, plan->bound, plan->vmax, &plan->low,
-                            plan->hi(), stream()),
+    check(algx_attn_forward_unit(ptr(q), ptr(k), ptr(v), fptr(s), unit, ptr(q_s), ptr(o),
+                                 fptr(o_precise), fptr(stat), static_cast<int32_t*>(ptr(guard)),
+                                 ptr(ws), ptr(bws), B, H, T, D, dtype_code(q), plan->scale,
+                                 plan->bound, plan->vmax, &plan->low, plan->hi(), stream()),
           "algx_attn_forward");
     ctx->save_for_backward({q_s, k, v, s, o, o_precise, stat, guard});
     ctx->saved_data["plan"] = at::IValue::make_capsule(plan);
@@ -167,16 +164,13 @@ struct Flash : Function<Flash> {
       ws = scratch(algx_attn_bwd_workspace_bytes(B, H, T, D), q_s);
       state = ALGX_ATTN_WS_RAW;
     }
-    check(algx_attn_bwd(ptr(q_s), ptr(k), ptr(v), fptr(s), ptr(o), fptr(o_precise), fptr(stat),
-                        ptr(dout), ptr(dq), ptr(dk), ptr(dv), fptr(dsink), ptr(ws), state, B, H, T,
-                        D, dtype_code(q_s), plan->scale, &plan->low, plan->hi(),
-                        static_cast<const int32_t*>(ptr(guard)), stream()),
+    check(algx_attn_bwd_unit(ptr(q_s), ptr(k), ptr(v), fptr(s), ctx->saved_data["unit"].toDouble(),
+                             ptr(o), fptr(o_precise), fptr(stat), ptr(dout), ptr(dq), ptr(dk),
+                             ptr(dv), fptr(dsink), ptr(ws), state, B, H, T, D, dtype_code(q_s),
+                             plan->scale, &plan->low, plan->hi(),
+                             static_cast<const int32_t*>(ptr(guard)), stream()),
           "algx_attn_bwd");
-    if (dsink.defined()) {
-      const double unit = ctx->saved_data["unit"].toDouble();
-      if (unit != 1.0) dsink = dsink.div(unit);
-      dsink = dsink.reshape(ctx->saved_data["sink_shape"].toIntVector());
-    }
+    if (dsink.defined()) dsink = dsink.reshape(ctx->saved_data["sink_shape"].toIntVector());
     return {dq, dk, dv, dsink, Tensor(), Tensor(), Tensor()};
   }
 };

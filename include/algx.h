@@ -161,6 +161,23 @@ int32_t algx_attn_forward(const void* q, const void* k, const void* v, const flo
                           const algx_attn_variant* low, const algx_attn_variant* high,
                           void* stream);
 
+/* algx_attn_forward and algx_attn_bwd with the sink (and its gradient) in
+ * units of sink_unit > 0: the kernels divide (flash.py:830-831), so a caller
+ * that holds the model's logits need not form the scaled array. */
+int32_t algx_attn_forward_unit(const void* q, const void* k, const void* v, const float* sink,
+                               float sink_unit, void* q_s, void* o, float* o_precise, float* stat,
+                               int32_t* guard, void* workspace, void* bwd_workspace, int32_t B,
+                               int32_t H, int32_t T, int32_t D, int32_t dtype, float q_scale,
+                               float bound, float vmax, const algx_attn_variant* low,
+                               const algx_attn_variant* high, void* stream);
+int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* v, const float* sink,
+                           float sink_unit, const void* o, const float* o_precise,
+                           const float* stat, const void* dout, void* dq, void* dk, void* dv,
+                           float* dsink, void* workspace, int32_t workspace_state, int32_t B,
+                           int32_t H, int32_t T, int32_t D, int32_t dtype, float q_scale,
+                           const algx_attn_variant* low, const algx_attn_variant* high,
+                           const int32_t* guard, void* stream);
+
 /* No counterpart in the reference: algx_attn_forward for callers that cannot
  * allocate (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc). Same arguments and results, no workspace: the guard's partial
