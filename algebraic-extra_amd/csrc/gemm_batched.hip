@@ -37,20 +37,16 @@ struct GemmGroups {
   int ngroups;
 };
 
-// Workgroup b -> (matrix, tile). Workgroups are dealt to the 8 XCDs
-// round-robin by index; when the batch is a multiple of 8, matrix j's tiles
-// go to indices congruent to j mod 8, i.e. all to one XCD and its L2, in
-// consecutive order there.
-__device__ __forceinline__ void batch_tile(int b, const BatchGemm& p, int& mat, int& tile) {
-  const int T = p.ntiles;
-  if (p.batch % 8 == 0) {
-    const int x = b & 7, r = b >> 3;  // XCD, index within it
-    mat = (r / T) * 8 + x;
-    tile = r % T;
-  } else {
-    mat = b / T;
-    tile = b % T;
-  }
+// Workgroup b -> (matrix, tile), false past the end. Workgroups are dealt to
+// the 8 XCDs round-robin by index; each XCD takes a run of consecutive units,
+// so a matrix's tiles run on one XCD and its L2 (two at a run's end), whatever
+// the batch.
+__device__ __forceinline__ bool batch_tile(int b, const BatchGemm& p, int& mat, int& tile) {
+  const int units = p.batch * p.ntiles;
+  const int unit = (b & 7) * ((units + 7) / 8) + (b >> 3);
+  mat = unit / p.ntiles;
+  tile = unit % p.ntiles;
+  return unit < units;
 }
 
 // Row-major index of tile (a, b), a <= b, of the upper triangle of t x t
@@ -132,9 +128,8 @@ __global__ __launch_bounds__(kThreads) void batched_gemm_kernel(GemmGroups gp) {
     if (i < gp.ngroups && (int)blockIdx.x >= gp.start[i]) gi = i;
   const BatchGemm p = gp.g[gi];
   const int local = (int)blockIdx.x - gp.start[gi];
-  if (local >= p.batch * p.ntiles) return;  // padding of the group to a multiple of 8
   int mat, tile;
-  batch_tile(local, p, mat, tile);
+  if (!batch_tile(local, p, mat, tile)) return;  // padding of the group to a multiple of 8
   int n0, m0;
   if (SYM) {
     int a, b;
