@@ -40,7 +40,9 @@ struct GemmGroups {
 // Workgroup b -> (matrix, tile), false past the end. Workgroups are dealt to
 // the 8 XCDs round-robin by index; each XCD takes a run of consecutive units,
 // so a matrix's tiles run on one XCD and its L2 (two at a run's end), whatever
-// the batch.
+// the batch. Dealing the tiles of a batch of 84 over all XCDs made every L2
+// fetch every operand: a X + B X of 48 x [768, 768] and 36 x [768, 2048] took
+// 261 us, 236 so (both with the register epilogue).
 __device__ __forceinline__ bool batch_tile(int b, const BatchGemm& p, int& mat, int& tile) {
   const int units = p.batch * p.ntiles;
   const int unit = (b & 7) * ((units + 7) / 8) + (b >> 3);
@@ -62,16 +64,15 @@ __device__ __forceinline__ void upper_tile(int idx, int t, int& a, int& b) {
   b = a + idx;
 }
 
-// C[m][n] (+ beta D) of a finished 256 x 256 tile of C^T at (n0, m0):
+// C[m][n] (+ beta D) of a finished 256 x 256 tile of C^T at (n0, m0) from
+// registers:
 // acc.v[i][j][4q + u] = C[m][n + u], m = m0 + WTN wn + 32 j + c32,
 // n = n0 + WTM wm + 32 i + 8 q + 4 g (N % 8 == 0: a run is whole or absent).
-// Each run's bf16 values also go to mirror(r, col, value4) when given. The
-// D runs of one j are all loaded before any is used (outside rows and
+// The D runs of one j are all loaded before any is used (outside rows and
 // columns read D's first run instead), so a lane waits for D once per j
 // rather than once per run.
-template <typename Mirror>
 __device__ __forceinline__ void store_tile(const BatchGemm& p, int mat, int m0, int n0,
-                                           const Acc& acc, int tid, Mirror&& mirror) {
+                                           const Acc& acc, int tid) {
   const int w = tid >> 6, lane = tid & 63, g = lane >> 5, c32 = lane & 31;
   const int wm = w / NWN, wn = w % NWN;
   bf16* C = p.C + mat * p.sc;
@@ -107,17 +108,117 @@ __device__ __forceinline__ void store_tile(const BatchGemm& p, int mat, int m0, 
         }
         const bf16x4 o = {(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
         *reinterpret_cast<bf16x4*>(C + (int64_t)m * p.ldc + n) = o;
-        mirror(n - n0, m - m0, o);
       }
+  }
+}
+
+// The same through the direct-to-LDS ring, idle after the k loop: each wave
+// owns 16 KB of it for its 64 rows (m) x 128 columns (n) of C, in 16-byte
+// chunks with chunk c of row r at c ^ (r & 15). D's rows come in by
+// direct-to-LDS loads, every lane combines its runs of four in place, and C
+// leaves in 256-byte row pieces. A mirrored (off-diagonal symmetric) tile then
+// goes through the same LDS as 128 rows (n) x 64 columns (m). No wave touches
+// another's part, so the one barrier is the caller's, between the k loop's last
+// reads of the ring and this.
+// From registers every D load and C store touched 32 rows, 16 bytes of each,
+// and took longer than the k loop of a 768-wide product. For 48 x [768, 768]
+// and 36 x [768, 2048]: a X + B X 235 -> 188 us, b A + c A A 90 -> 74, the Gram
+// products (no D) 105 both ways; for 16 x [1024, 1024] and 12 x [1024, 2688]
+// 176 -> 144, 88 -> 73 and 87 -> 82. What bounds the short products now is the
+// traffic of a tile's operands, D and C, which the one workgroup of a compute
+// unit does not overlap with its k loop.
+// 256 rows of D stay within the loads' 32-bit byte offsets; wider ones take the
+// register-staged kernel.
+constexpr int64_t kMaxLdd = int64_t(1) << 22;
+__device__ __forceinline__ void store_tile_lds(const BatchGemm& p, int mat, int m0, int n0,
+                                               Acc& acc, bool mirror, const DmaRing& ring,
+                                               int tid) {
+  static_assert(WTM == 128 && WTN == 64 && kDmaStages >= 4, "16 KB of the ring per wave");
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, g = lane >> 5, c32 = lane & 31;
+  const int wm = w / NWN, wn = w % NWN;
+  const int mr = m0 + WTN * wn, nc = n0 + WTM * wm;  // the wave's first row and column
+  bf16* const slot = (w >> 1) == 0   ? ring.slot[0]
+                     : (w >> 1) == 1 ? ring.slot[1]
+                     : (w >> 1) == 2 ? ring.slot[2]
+                                     : ring.slot[3];
+  bf16* const part = slot + (w & 1) * (WTM * WTN);
+  const bool has_d = p.D != nullptr;
+  if (has_d) {
+    // Offsets count from the tile's first element, which is inside D; pieces
+    // outside D read that element's piece and are not used.
+    const bf16* base = p.D + mat * p.sd + (int64_t)m0 * p.ldd + n0;
+    const unsigned lds = lds_addr(part);
+#pragma unroll
+    for (int b = 0; b < WTN / 4; ++b) {
+      const int r = 4 * b + (lane >> 4), c = (lane & 15) ^ (r & 15);
+      const bool in = mr + r < p.M && nc + 8 * c < p.N;
+      const unsigned at = (unsigned)(WTN * wn + r) * (unsigned)p.ldd + (WTM * wm + 8 * c);
+      dma16s(base, in ? 2u * at : 0u, lds + 1024u * b);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+#pragma unroll
+  for (int j = 0; j < TJ; ++j)
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = 32 * j + c32;
+        bf16x4* at =
+            reinterpret_cast<bf16x4*>(part + r * WTM + 8 * ((4 * i + q) ^ (r & 15)) + 4 * g);
+        f32x4 v;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = p.alpha * acc.v[i][j][4 * q + u];
+        if (has_d) {
+          const bf16x4 d = *at;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = __builtin_fmaf(p.beta, (float)d[u], v[u]);
+        }
+        *at = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc.v[i][j][4 * q + u] = v[u];
+      }
+  asm volatile("" ::: "memory");  // a wave's LDS operations complete in order
+  bf16* const C = p.C + mat * p.sc;
+#pragma unroll
+  for (int b = 0; b < WTN / 4; ++b) {
+    const int r = 4 * b + (lane >> 4), pos = lane & 15;
+    const int m = mr + r, n = nc + 8 * (pos ^ (r & 15));
+    if (m < p.M && n < p.N)
+      *reinterpret_cast<bf16x8*>(C + (int64_t)m * p.ldc + n) =
+          *reinterpret_cast<const bf16x8*>(part + r * WTM + 8 * pos);
+  }
+  if (!mirror) return;
+  asm volatile("" ::: "memory");
+  // C[n][m] = C[m][n]; chunk c of row r at c ^ 4 ((r >> 2) & 1), so the two
+  // lane halves (rows four apart) write different banks.
+#pragma unroll
+  for (int j = 0; j < TJ; ++j)
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int r = 32 * i + 8 * (e >> 2) + 4 * g + (e & 3);
+        part[r * WTN + ((32 * j + c32) ^ (32 * g))] = (bf16)acc.v[i][j][e];
+      }
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int b = 0; b < WTM / 8; ++b) {
+    const int r = 8 * b + (lane >> 3), pos = lane & 7;
+    const int n = nc + r, m = mr + 8 * (pos ^ (4 * ((r >> 2) & 1)));
+    if (n < p.N && m < p.M)
+      *reinterpret_cast<bf16x8*>(C + (int64_t)n * p.ldc + m) =
+          *reinterpret_cast<const bf16x8*>(part + r * WTN + 8 * pos);
   }
 }
 
 // Each workgroup forms a 256 x 256 tile of C^T (the kernel's M axis runs
 // over C's columns n, its N axis over C's rows m), so every lane holds runs
-// of four consecutive columns of one row: C and D move in 8-byte pieces.
+// of four consecutive columns of one row.
 // SYM (C symmetric, M == N, D symmetric when present): only the tiles on and
 // above the diagonal are formed; an off-diagonal tile's values also go to
-// the mirrored tile, transposed through the idle stage buffers.
+// the mirrored tile.
 template <bool AKC, bool BKC, bool DMA, bool SYM>
 __global__ __launch_bounds__(kThreads) void batched_gemm_kernel(GemmGroups gp) {
   GEMM_LDS_STAGES;
@@ -147,32 +248,12 @@ __global__ __launch_bounds__(kThreads) void batched_gemm_kernel(GemmGroups gp) {
     gemm_tile_dma<BKC, AKC>(Bop, Aop, n0, m0, ring, acc, tid);
   else
     gemm_tile<BKC, AKC>(Bop, Aop, n0, m0, s0, s0 + 2 * kStageElems, acc, tid);
-  const bool mirror = SYM && m0 != n0;  // uniform over the workgroup
-  // stage buffer k of the ring (constant indices only: a runtime index would
-  // place the ring in a static initializer)
-  auto buf = [&](int k) -> bf16* {
-    return k == 0 ? ring.slot[0] : k == 1 ? ring.slot[1] : k == 2 ? ring.slot[2] : ring.slot[3];
-  };
-  static_assert(!SYM || DMA, "the mirrored tile is staged in the four 32 KB stage buffers");
-  // every wave's last LDS reads of the k loop are done before staging
-  if (mirror) __syncthreads();
-  store_tile(p, mat, m0, n0, acc, tid, [&](int r, int col, const bf16x4& o) {
-    // row r + u of the mirrored tile (256 columns m), 64 rows per stage buffer
-    if (mirror) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) buf((r + u) >> 6)[((r + u) & 63) * BN + col] = o[u];
-    }
-  });
-  bf16* C = p.C + mat * p.sc;
-  if (mirror) {
-    __syncthreads();
-    // C[n][m] = C[m][n] for the staged rows, 16-byte pieces (M % 8 == 0)
-    for (int c = tid; c < BM * BN / 8; c += kThreads) {
-      const int r = c / (BN / 8), col = 8 * (c % (BN / 8));
-      if (n0 + r < p.M && m0 + col < p.M)
-        *reinterpret_cast<bf16x8*>(C + (int64_t)(n0 + r) * p.ldc + m0 + col) =
-            *reinterpret_cast<const bf16x8*>(buf(r >> 6) + (r & 63) * BN + col);
-    }
+  static_assert(!SYM || DMA, "the mirrored tile is staged in the ring");
+  if constexpr (DMA) {
+    __syncthreads();  // every wave's last LDS reads of the k loop are done
+    store_tile_lds(p, mat, m0, n0, acc, SYM && m0 != n0, ring, tid);
+  } else {
+    store_tile(p, mat, m0, n0, acc, tid);
   }
 }
 
@@ -414,7 +495,8 @@ int32_t launch_groups(const algx_gemm_batch* groups, int ngroups, bool a_kc, boo
     if (p.batch == 0 || p.M == 0 || p.N == 0) continue;
     // (the kernel's A is the caller's B and vice versa)
     if (p.K % BK == 0 && dma_span_ok(Operand{nullptr, p.ldb, p.N, p.K}, b_kc) &&
-        dma_span_ok(Operand{nullptr, p.lda, p.M, p.K}, a_kc))
+        dma_span_ok(Operand{nullptr, p.lda, p.M, p.K}, a_kc) &&
+        (p.D == nullptr || p.ldd <= kMaxLdd))
       dma[nd++] = p;
     else
       reg[nr++] = p;

@@ -278,6 +278,27 @@ def test_operands_beyond_32bit_lane_offsets_take_the_staged_path():
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("ldd", [80, 1 << 22, (1 << 22) + 8])
+def test_combined_matrix_of_any_row_stride(ldd):
+    """D's rows up to 2^22 elements apart come in by direct-to-LDS loads, wider
+    ones through registers; both equal the dense D bit for bit. Ragged tiles
+    in both directions, D's last row ending its allocation."""
+    from algebraic_amd import _lib
+    M, N, K = 264, 72, 64
+    g = torch.Generator(device=DEV).manual_seed(22)
+    A = torch.randn((1, M, K), generator=g, device=DEV).bfloat16()
+    B = torch.randn((1, N, K), generator=g, device=DEV).bfloat16()
+    D = torch.randn((1, M, N), generator=g, device=DEV).bfloat16()
+    want = O.gemm_bf16_batched(A, B, a_kc=True, b_kc=True, D=D, alpha=-0.5, beta=1.5)
+    wide = torch.empty(((M - 1) * ldd + N,), device=DEV, dtype=torch.bfloat16)
+    wide.as_strided((M, N), (ldd, 1)).copy_(D[0])
+    C = torch.full((1, M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    _lib.call("algx_gemm_bf16_batched", _lib.ptr(A), _lib.ptr(B), _lib.ptr(wide), _lib.ptr(C), 1,
+              M, N, K, 1, 1, 0, K, K, ldd, N, 0, 0, 0, 0, -0.5, 1.5, _lib.stream())
+    assert torch.equal(C, want)
+    _check(C, _ref(A, B, True, True, D, -0.5, 1.5))
+
+
 @pytest.mark.parametrize("T,din,dout", [(1, 8, 8), (31, 264, 40), (33, 256, 512), (1000, 384, 1152),
                                         (2055, 1032, 520), (8192, 768, 2304), (4096, 1024, 5376)])
 def test_weight_grad_any_token_count(T, din, dout):
