@@ -148,13 +148,8 @@ extern "C" int32_t algx_attn_fwd(const void* q, const void* k, const void* v, co
   hipStream_t s = (hipStream_t)stream;
   if (mfma_supported(T, D, dtype) && !force_generic())
     return launch_fwd_mfma(q, k, v, sink, o, o_precise, stat, B, H, T, kl, kh, guard, s);
-  if (int32_t rc = launch_fwd_generic(q, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kl,
-                                      guard, 1, s))
-    return rc;
-  if (guard != nullptr)
-    return launch_fwd_generic(q, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kh, guard, 0,
-                              s);
-  return 0;
+  return launch_fwd_generic(q, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kl, kh, guard,
+                            s);
 }
 
 extern "C" int64_t algx_attn_forward_workspace_bytes(int32_t B, int32_t H, int32_t T,
@@ -207,13 +202,8 @@ extern "C" int32_t algx_attn_forward_unit(const void* q, const void* k, const vo
   if (int32_t rc = launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound,
                                   vmax, sink_unit, s))
     return rc;
-  if (int32_t rc = launch_fwd_generic(q_s, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kl,
-                                      guard, 1, s))
-    return rc;
-  if (guard != nullptr)
-    return launch_fwd_generic(q_s, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kh, guard,
-                              0, s);
-  return 0;
+  return launch_fwd_generic(q_s, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kl, kh, guard,
+                            s);
 }
 
 extern "C" int32_t algx_attn_forward(const void* q, const void* k, const void* v,
@@ -292,13 +282,8 @@ extern "C" int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* 
   }
   if (sg.dsink != nullptr)
     if (int32_t rc = launch_sink_finish(sg, s)) return rc;
-  if (int32_t rc = launch_bwd_generic(q, k, v, stat, di, dout, dq, dk, dv, B, H, T, D, dtype,
-                                      q_scale, kl, guard, 1, s))
-    return rc;
-  if (guard != nullptr)
-    return launch_bwd_generic(q, k, v, stat, di, dout, dq, dk, dv, B, H, T, D, dtype, q_scale, kh,
-                              guard, 0, s);
-  return 0;
+  return launch_bwd_generic(q, k, v, stat, di, dout, dq, dk, dv, B, H, T, D, dtype, q_scale, kl,
+                            kh, guard, s);
 }
 
 extern "C" int32_t algx_attn_bwd(const void* q, const void* k, const void* v, const float* sink,

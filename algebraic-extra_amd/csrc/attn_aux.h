@@ -37,15 +37,16 @@ int32_t launch_dq_finish(const float* acc, void* dq, int64_t heads, int T, int D
                          const KVariant& low, const KVariant& high, const int32_t* guard,
                          float q_scale, const SinkGrad& sg, hipStream_t s);
 
-// Generic kernels: any T, D in {16, 32, 64}, bf16 or f32, every variant.
+// Generic kernels: any T, D in {16, 32, 64}, bf16 or f32, every variant. With a
+// guard word they run `lo` or `hi` for the whole call, else `lo`.
 int32_t launch_fwd_generic(const void* q_s, const void* k, const void* v, const float* sink,
                            void* o, float* o_precise, float* stat, int B, int H, int T, int D,
-                           int dtype, const KVariant& var, const int32_t* guard, int want_low,
+                           int dtype, const KVariant& lo, const KVariant& hi, const int32_t* guard,
                            hipStream_t s);
 int32_t launch_bwd_generic(const void* q, const void* k, const void* v, const float* stat,
                            const float* di, const void* dout, void* dq, void* dk, void* dv,
                            int B, int H, int T, int D, int dtype, float q_scale,
-                           const KVariant& var, const int32_t* guard, int want_low,
+                           const KVariant& lo, const KVariant& hi, const int32_t* guard,
                            hipStream_t s);
 
 // MFMA kernels: bf16, D = 64, any T.

@@ -25,9 +25,11 @@
 // per wave in flight, a wave loads the next tile's operands before the current
 // tile's products. Measured against the one-thread-per-row kernels these
 // replace (whose chains of D FMAs per score left all but a few CUs idle),
-// float32 guarded calls (two launches each, one of which returns at once):
-// forward B=1, H=4, T=256 287 -> 13 us; B=2, H=12, T=512 forward 575 -> 33 us,
-// backward 1223 -> 108 us. The distance from float64 did not grow (5.9e-7 ->
+// float32 guarded calls: forward B=1, H=4, T=256 287 -> 13 us; B=2, H=12, T=512
+// forward 575 -> 33 us, backward 1223 -> 108 us (with a second launch per kernel
+// for the variant the guard does not take, which returned at once; the kernels
+// now choose the variant themselves, and the first call as a whole went from 21
+// to 18 us). The distance from float64 did not grow (5.9e-7 ->
 // 5.6e-7 of o at the first shape).
 #include "attn_aux.h"
 
@@ -164,9 +166,9 @@ template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void fwd_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const float* __restrict__ sink, T* __restrict__ o, float* __restrict__ o_precise,
-    float* __restrict__ stat, int H, int T_, KVariant var, const int32_t* __restrict__ guard,
-    int want_low) {
-  if (guard != nullptr && (int)guard_in_range(guard) != want_low) return;
+    float* __restrict__ stat, int H, int T_, KVariant lo, KVariant hi,
+    const int32_t* __restrict__ guard) {
+  const KVariant var = guard_in_range(guard) ? lo : hi;
   __shared__ float acc_s[kWaves][kRows][D + 4];
   __shared__ float m_s[kWaves][kRows], l_s[kWaves][kRows];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -288,9 +290,9 @@ template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void bwd_dkdv_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const float* __restrict__ stat, const float* __restrict__ di, const T* __restrict__ dout,
-    T* __restrict__ dk, T* __restrict__ dv, int T_, KVariant var,
-    const int32_t* __restrict__ guard, int want_low) {
-  if (guard != nullptr && (int)guard_in_range(guard) != want_low) return;
+    T* __restrict__ dk, T* __restrict__ dv, int T_, KVariant lo,
+    KVariant hi, const int32_t* __restrict__ guard) {
+  const KVariant var = guard_in_range(guard) ? lo : hi;
   __shared__ float dk_s[kWaves][kRows][D + 4], dv_s[kWaves][kRows][D + 4];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int bh = blockIdx.y, kb = blockIdx.x;  // most queries first
@@ -367,9 +369,9 @@ template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void bwd_dq_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const float* __restrict__ stat, const float* __restrict__ di, const T* __restrict__ dout,
-    T* __restrict__ dq, int T_, float q_scale, KVariant var, const int32_t* __restrict__ guard,
-    int want_low) {
-  if (guard != nullptr && (int)guard_in_range(guard) != want_low) return;
+    T* __restrict__ dq, int T_, float q_scale, KVariant lo, KVariant hi,
+    const int32_t* __restrict__ guard) {
+  const KVariant var = guard_in_range(guard) ? lo : hi;
   __shared__ float dq_s[kWaves][kRows][D + 4];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int bh = blockIdx.y, qb = gridDim.x - 1 - blockIdx.x;
@@ -428,13 +430,13 @@ __global__ __launch_bounds__(kThreads) void bwd_dq_generic_kernel(
 
 int32_t launch_fwd_generic(const void* q, const void* k, const void* v, const float* sink,
                            void* o, float* o_precise, float* stat, int B, int H, int T, int D,
-                           int dtype, const KVariant& var, const int32_t* guard, int want_low,
+                           int dtype, const KVariant& lo, const KVariant& hi, const int32_t* guard,
                            hipStream_t s) {
   dim3 grid((T + kRows - 1) / kRows, B * H);
 #define FWD_CASE(TT, DD)                                                                         \
   fwd_generic_kernel<TT, DD><<<grid, kThreads, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, \
-                                                       sink, (TT*)o, o_precise, stat, H, T, var, \
-                                                       guard, want_low)
+                                                       sink, (TT*)o, o_precise, stat, H, T, lo,  \
+                                                       hi, guard)
   if (dtype == ALGX_BF16) {
     if (D == 64) FWD_CASE(bf16, 64);
     else if (D == 32) FWD_CASE(bf16, 32);
@@ -453,18 +455,18 @@ int32_t launch_fwd_generic(const void* q, const void* k, const void* v, const fl
 int32_t launch_bwd_generic(const void* q, const void* k, const void* v, const float* stat,
                            const float* di, const void* dout, void* dq, void* dk, void* dv,
                            int B, int H, int T, int D, int dtype, float q_scale,
-                           const KVariant& var, const int32_t* guard, int want_low,
+                           const KVariant& lo, const KVariant& hi, const int32_t* guard,
                            hipStream_t s) {
   dim3 grid((T + kRows - 1) / kRows, B * H);
 #define BWD_CASE(TT, DD)                                                                        \
   do {                                                                                          \
     bwd_dkdv_generic_kernel<TT, DD><<<grid, kThreads, 0, s>>>(                                  \
         (const TT*)q, (const TT*)k, (const TT*)v, stat, di, (const TT*)dout, (TT*)dk, (TT*)dv, \
-        T, var, guard, want_low);                                                               \
+        T, lo, hi, guard);                                                                      \
     bwd_dq_generic_kernel<TT, DD><<<grid, kThreads, 0, s>>>((const TT*)q, (const TT*)k,         \
                                                             (const TT*)v, stat, di,             \
                                                             (const TT*)dout, (TT*)dq, T,        \
-                                                            q_scale, var, guard, want_low);     \
+                                                            q_scale, lo, hi, guard);            \
   } while (0)
   if (dtype == ALGX_BF16) {
     if (D == 64) BWD_CASE(bf16, 64);
