@@ -255,9 +255,13 @@ __global__ __launch_bounds__(256) void head_stat_kernel(HeadStat p) {
         tel = st - z;
         term = tel;
       } else {
-        const float x = __builtin_fminf(z * p.inv_c, p.clamp);
+        // A comparison, not a minimum: a NaN logit stays NaN, and so do the
+        // objective and a trainer's check of it. -inf becomes NaN (x - x), as
+        // the same expression on materialised logits gives.
+        float x = z * p.inv_c;
+        x = x > p.clamp ? p.clamp : x;
         const float r = __builtin_fabsf(x) + __builtin_sqrtf(__builtin_fmaf(x, x, 1.0f));
-        tel = pow2n((x >= 0.0f ? r : 1.0f / r) * st, p.log2n);
+        tel = pow2n((x >= 0.0f ? r : 1.0f / r) * st, p.log2n) + (x - x);
         term = 1.0f - tel;
       }
       p.tel[t] = tel;

@@ -101,3 +101,27 @@ def test_loss_over_token_blocks(N, dtype):
     # float32 sums of 3001 terms: 1e-6 relative, and one rounding of lse - zt
     np.testing.assert_allclose(to_np(tel), lse - zt, rtol=1e-5, atol=1e-5)
     np.testing.assert_allclose(float(obj), (lse - zt).mean(), rtol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["ce", "alg_ce"])
+@pytest.mark.parametrize("bad", ["nan", "minus_inf"])
+def test_non_finite_target_logit_reaches_the_objective(dtype, kind, bad):
+    """A target logit that is NaN (a NaN hidden state) or -inf gives NaN for the
+    token and for the objective, so that a trainer stops on it, as the formula
+    on materialised logits does; the other tokens keep their values."""
+    N, d, V, row = 70, 64, 513, 66
+    h, e, t = _head_inputs(N, d, V, 11, 0.2)
+    h, e, t = h.to(DEV, dtype), e.to(DEV, dtype), t.to(DEV)
+    e[:, 0] = 1.0
+    e[t[row], 0] = -1.0
+    kw = dict(kind=kind, n=8, c=2.0, block_n=N)
+    _, want = fused_head(h, e, t, **kw)
+    if bad == "nan":
+        h[row] = float("nan")
+    else:
+        h[row, 0] = float("inf")
+    obj, tel = fused_head(h, e, t, **kw)
+    others = torch.arange(N, device=DEV) != row
+    assert torch.equal(tel[others], want[others])
+    assert torch.isnan(tel[row]) and torch.isnan(obj)
