@@ -232,7 +232,9 @@ __global__ __launch_bounds__(kThreads) void fwd_generic_kernel(
       for (int i = 0; i < 4; ++i) {
         p[i] = var.kind == ALGX_SOFTMAX ? __expf(s[i] - m_new)
                                         : pow2n(rho_var(s[i], var.fast, r) * shf, var.log2n);
-        if (diag && 4 * g + i > c) p[i] = 0.0f;
+        // A score of -inf weighs nothing, also where the wave has met no other
+        // score yet (m_new = -inf): a row is NaN only if all its scores are.
+        if ((diag && 4 * g + i > c) || s[i] == -__builtin_inff()) p[i] = 0.0f;
         lsum += p[i];
       }
       l = l * alpha + lsum;

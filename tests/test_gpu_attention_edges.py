@@ -114,3 +114,41 @@ def test_generic_later_rows_stay_apart(kw):
     assert rel_l2(dq[0, 0, :j], g_ref[0][0, 0, :j]) <= 1e-6
     assert rel_l2(dv[0, 0, j + 1:], g_ref[2][0, 0, j + 1:]) <= 1e-6
     assert rel_l2(dk[0, 0, j + 1:], g_ref[1][0, 0, j + 1:]) <= 1e-6
+
+
+@pytest.mark.parametrize("D,dtype", [(64, "f32"), (32, "f32"), (16, "bf16")])
+@pytest.mark.parametrize("kw", [dict(kind="softmax"),
+                                dict(kind="asinh", n=16, c=8.0, shift=True, fast_rho=False)],
+                         ids=["softmax", "shift"])
+def test_minus_infinite_scores(D, dtype, kw):
+    """Scores of -inf (finite inputs whose product overflows) weigh nothing: a
+    single key on the diagonal of a 16-row tile, a whole tile, a row's first
+    tiles and all but one key. Such a row has no maximum yet where a wave meets
+    nothing else first. Against float64, where the weights are exactly 0."""
+    T, big = 130, 1e30
+    pairs = {16: [16], 31: range(16, 32), 50: range(0, 16), 90: range(0, 90), 129: range(64, 130)}
+    q, k, v, g = (x.cuda().float() for x in _rand((1, 1, T, D), 29, dtype="f32"))
+    q[..., 0] = k[..., 0] = 0.0
+    out = []
+    for i, js in pairs.items():     # one query at a time: its keys hold the large value
+        qi, ki = q.clone(), k.clone()
+        qi[0, 0, i, 0] = -big
+        ki[0, 0, list(js), 0] = big
+        dt = torch.float32 if dtype == "f32" else torch.bfloat16
+        leaves = [x.to(dt).requires_grad_() for x in (qi, ki, v)]
+        o = flash_attention(*leaves, block=T, **kw)
+        ref = [x.detach().double().requires_grad_() for x in leaves]
+        s = ref[0] @ ref[1].transpose(-1, -2) / D ** 0.5
+        if kw["kind"] == "asinh":
+            s = kw["n"] * torch.asinh(s / kw["c"])
+        p = torch.softmax(s.masked_fill(torch.ones(T, T, device=s.device).triu(1) > 0,
+                                        -float("inf")), -1)
+        want = p @ ref[2]
+        tol = 1e-5 if dtype == "f32" else 1e-2      # float32 sums; bf16 weights and output
+        assert torch.isfinite(o).all(), (i, js)
+        assert rel_l2(o, want) <= tol, (i, js)
+        if kw["kind"] == "softmax":
+            got = torch.autograd.grad(o, leaves, g.to(dt))
+            exp = torch.autograd.grad(want, ref, g.to(dt).double())
+            for a, b, name in zip(got, exp, "qkv"):
+                assert rel_l2(a[..., 1:], b[..., 1:]) <= (1e-4 if dtype == "f32" else 2e-2), name
