@@ -79,6 +79,11 @@ bool force_generic() {
   return e != nullptr && e[0] == '1';
 }
 
+// Whether the MFMA kernels run the call; pair: they have its variants.
+bool use_mfma(int T, int D, int dtype, bool pair) {
+  return mfma_supported(T, D, dtype) && (whole_blocks(T) || pair) && !force_generic();
+}
+
 // The kernels move (B, H, T, D) rows with 16-byte vector accesses.
 int32_t check_aligned(const char* who, std::initializer_list<const void*> ptrs) {
   for (const void* p : ptrs)
@@ -146,7 +151,7 @@ extern "C" int32_t algx_attn_fwd(const void* q, const void* k, const void* v, co
     return fail("attn_fwd: precise-output variant needs o_precise");
   if (int32_t rc = check_aligned("attn_fwd", {q, k, v, o, o_precise})) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (mfma_supported(T, D, dtype) && !force_generic())
+  if (use_mfma(T, D, dtype, mfma_pair(kl, kh)))
     return launch_fwd_mfma(q, k, v, sink, o, o_precise, stat, B, H, T, kl, kh, guard, s);
   return launch_fwd_generic(q, k, v, sink, o, o_precise, stat, B, H, T, D, dtype, kl, kh, guard,
                             s);
@@ -187,17 +192,17 @@ extern "C" int32_t algx_attn_forward_unit(const void* q, const void* k, const vo
   hipStream_t s = (hipStream_t)stream;
   // A guarded call without a workspace for the partial maxima takes the
   // generic path where T is no multiple of the MFMA path's query block.
-  const bool mfma = mfma_supported(T, D, dtype) && !force_generic();
   const bool parts = guard == nullptr || workspace != nullptr;
-  if (mfma && (parts || whole_blocks(T))) {
+  const bool pair = guard == nullptr || mfma_fused_pair(kl, kh);
+  if (use_mfma(T, D, dtype, pair && parts)) {
     if (!parts) return fail("attn_forward: the guard needs the workspace");
     // The backward workspace starts with its float32 dQ accumulator.
     return launch_fwd_fused(q, k, v, sink, q_s, o, o_precise, stat, guard, (float*)workspace,
                             (float*)bwd_workspace, B, H, T, q_scale, bound, vmax, kl, kh, s);
   }
-  // The backward of such a call still runs MFMA and finds its accumulator
+  // The backward of such a call may still run MFMA and finds its accumulator
   // cleared.
-  if (mfma && bwd_workspace != nullptr)
+  if (bwd_workspace != nullptr && use_mfma(T, D, dtype, mfma_pair(kl, kh)))
     if (int32_t rc = fill_f32((float*)bwd_workspace, acc_bytes(B, H, T, D) / 4, 0.0f, s)) return rc;
   if (int32_t rc = launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound,
                                   vmax, sink_unit, s))
@@ -259,7 +264,7 @@ extern "C" int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* 
     return fail("attn_bwd: precise-output variant needs o_precise");
   if (int32_t rc = check_aligned("attn_bwd", {q, k, v, o, o_precise, dout, dq, dk, dv, workspace}))
     return rc;
-  const bool mfma = mfma_supported(T, D, dtype) && !force_generic();
+  const bool mfma = use_mfma(T, D, dtype, mfma_pair(kl, kh));
   float* dq_acc = (float*)workspace;
   float* di = (float*)((char*)workspace + acc_bytes(B, H, T, D));
   // The pre-pass forms di and the shares of dsink, and clears the dQ

@@ -51,6 +51,12 @@ int32_t launch_bwd_generic(const void* q, const void* k, const void* v, const fl
 
 // MFMA kernels: bf16, D = 64, any T.
 bool mfma_supported(int T, int D, int dtype);
+// Whether they have the variant pair of a guarded call: one launch for both
+// (algx_attn_fwd, the backward), or the fused forward's two. Without it the
+// generic kernels run at T that is no multiple of 128, as for any variants
+// there; other T have no other kernels and are refused.
+bool mfma_pair(const KVariant& lo, const KVariant& hi);
+bool mfma_fused_pair(const KVariant& lo, const KVariant& hi);
 // Rows per head of the MFMA backward's float32 dQ accumulator: T rounded up to
 // whole 128-row query blocks, so that the forward clears and the backward adds
 // whole blocks.

@@ -9,6 +9,14 @@ bool mfma_supported(int T, int D, int dtype) {
   return dtype == ALGX_BF16 && D == mfma::HD && T > 0;
 }
 
+bool mfma_pair(const KVariant& lo, const KVariant& hi) {
+  return mfma::pair_ok(mfma::cfg_for(lo), mfma::cfg_for(hi));
+}
+
+bool mfma_fused_pair(const KVariant&, const KVariant& hi) {
+  return mfma::high_ok(mfma::cfg_for(hi));
+}
+
 int64_t fwd_fused_partials(int B, int H, int T) {
   return (int64_t)B * H * ((T + mfma::FBM - 1) / mfma::FBM);
 }

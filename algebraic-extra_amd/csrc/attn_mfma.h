@@ -79,6 +79,15 @@ inline int cfg_for(const KVariant& v) {
   return cfg_of(MODE_NOSHIFT, v.fast != 0, v.bounded != 0, l2n_arg(v.log2n));
 }
 
+// Guarded launches pair a bounded unshifted low variant with the shifted
+// exact-rho high variant of the same n (flash.py:850-852): the pairs of
+// ALGX_PICK_ALL, and the high variants of the fused forward's second launch.
+inline bool high_ok(int ch) { return ch == cfg_of(MODE_SHIFT, false, false, cfg_l2n(ch)); }
+inline bool pair_ok(int cl, int ch) {
+  return cl == ch || (cfg_mode(cl) == MODE_NOSHIFT && cfg_bounded(cl) && !cfg_poly(cl) &&
+                      high_ok(ch) && cfg_l2n(cl) == cfg_l2n(ch));
+}
+
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -165,8 +174,7 @@ template <int L2N> __device__ __forceinline__ float powN(float x, int log2n) {
 
 #define ALGX_PICK_SINGLE(K, C) \
   if (cl == (C)) return K<(C), (C)>;
-// Guarded launches pair a bounded unshifted low variant with the shifted
-// exact-rho high variant of the same n (flash.py:850-852).
+// Guarded launches: the pairs of pair_ok.
 #define ALGX_PICK_GUARDED(K, FASTLO, L2)                                                    \
   if (cl == cfg_of(MODE_NOSHIFT, FASTLO, true, L2) && ch == cfg_of(MODE_SHIFT, false, false, L2)) \
     return K<cfg_of(MODE_NOSHIFT, FASTLO, true, L2), cfg_of(MODE_SHIFT, false, false, L2)>;

@@ -4,11 +4,15 @@ Tolerances as in tests/_tol.py; the sink gradient, a float32 sum over batch
 and rows of terms formed from the storage dtype, as in test_gpu_attention.py.
 """
 
+import math
+
 import pytest
 import torch
 
 from _tol import rel_l2
+from algebraic_amd import _lib
 from algebraic_amd.kernels import flash_attention
+from algebraic_amd.kernels.flash import _c_variant, make_variant
 from test_gpu_attention import _check_all, _oracle, _rand, _run
 
 pytestmark = pytest.mark.gpu
@@ -152,3 +156,57 @@ def test_minus_infinite_scores(D, dtype, kw):
             exp = torch.autograd.grad(want, ref, g.to(dt).double())
             for a, b, name in zip(got, exp, "qkv"):
                 assert rel_l2(a[..., 1:], b[..., 1:]) <= (1e-4 if dtype == "f32" else 2e-2), name
+
+
+def _abi(q, k, v, do, lo, hi=None, guard=None, fused=False):
+    """o, dq, dk, dv of the C ABI calls for the given variants: the forward
+    alone on a guard word set by the caller, or (fused) as one call that forms
+    the word (bounds that every input keeps)."""
+    B, H, T, D = q.shape
+    dt, st, p = _lib.dtype_code(q.dtype), _lib.stream(), _lib.ptr
+    scale = 1.0 / (8.0 * math.sqrt(D))
+    q_s, o, dq, dk, dv = (torch.empty_like(q) for _ in range(5))
+    o_precise = torch.empty(q.shape, dtype=torch.float32, device="cuda")
+    stat = torch.empty((B, H, T), dtype=torch.float32, device="cuda")
+    ws = torch.empty(_lib.query("algx_attn_forward_workspace_bytes", B, H, T, D),
+                     dtype=torch.uint8, device="cuda")
+    bws = torch.empty(_lib.query("algx_attn_bwd_workspace_bytes", B, H, T, D),
+                      dtype=torch.uint8, device="cuda")
+    word = None
+    if guard is not None:
+        word = torch.zeros(_lib.query("algx_attn_guard_words"), dtype=torch.int32, device="cuda")
+        word[0] = guard
+    if fused:
+        _lib.call("algx_attn_forward", p(q), p(k), p(v), None, p(q_s), p(o), p(o_precise), p(stat),
+                  p(word), p(ws), p(bws), B, H, T, D, dt, scale, 1e9 if guard else 0.0, 1e9, lo,
+                  hi, st)
+    else:
+        _lib.call("algx_attn_prepare", p(q), p(k), p(v), None, p(q_s), None, B, H, T, D, dt, scale,
+                  0.0, 0.0, st)
+        _lib.call("algx_attn_fwd", p(q_s), p(k), p(v), None, p(o), p(o_precise), p(stat), B, H, T,
+                  D, dt, lo, hi, p(word), st)
+    _lib.call("algx_attn_bwd", p(q_s), p(k), p(v), None, p(o), p(o_precise), p(stat), p(do), p(dq),
+              p(dk), p(dv), None, p(bws), _lib.ATTN_WS_CLEARED if fused else _lib.ATTN_WS_RAW, B, H,
+              T, D, dt, scale, lo, hi, p(word), st)
+    torch.cuda.synchronize()
+    if word is not None:
+        assert int(word[0]) == guard
+    return o, dq, dk, dv
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("guard", [0, 1])
+def test_ragged_takes_any_variant_pair(guard, fused):
+    """The C ABI's guarded calls pair any two variants at lengths that are no
+    multiple of 128: pairs that the MFMA kernels do not have, against the chosen
+    variant alone."""
+    T = 77
+    q, k, v, g = (x.cuda() for x in _rand((2, 3, T, 64), 41))
+    shift = _c_variant(make_variant("asinh", 16, 8.0, T, shift=True, fast_rho=False))
+    clamped = _c_variant(make_variant("asinh", 16, 8.0, T, shift=False))
+    softmax = _c_variant(make_variant("softmax"))
+    for lo, hi in ((shift, clamped), (clamped, shift), (softmax, shift)):
+        got = _abi(q, k, v, g, lo, hi, guard, fused)
+        want = _abi(q, k, v, g, lo if guard else hi)
+        for a, b, name in zip(got, want, ("o", "dq", "dk", "dv")):
+            assert rel_l2(a, b) <= 1e-2, name       # bf16 weights and outputs
