@@ -27,9 +27,11 @@
 // query's statistic makes its weights zero, such a key lies above the diagonal
 // of every query that counts, and the dQ accumulator has whole 128-row blocks
 // per head, so only the tile loader tests bounds. (One kernel for both cost
-// the B=8, H=16, T=2048 layer about 1 %.) At B=2, H=12, T=333 the
-// one-thread-per-row kernels these replace there took 846 us of a guarded call
-// (two launches each); these take 28.0 us.
+// the B=8, H=16, T=2048 layer about 1 %.) di is subtracted in float32 there, as
+// by the kernels that ran these lengths before, not as two bf16 values: with
+// di near 257 and dP - di near 0.02 the two values left dq 8 % off. At B=2,
+// H=12, T=333 the one-thread-per-row kernels these replace there took 846 us of
+// a guarded call (two launches each); these take 28.0 us.
 #pragma once
 
 #include <type_traits>
@@ -226,7 +228,8 @@ __device__ __forceinline__ void bwd_body(
     L.dd[buf][lane] = pdi;
   };
 
-  // S and dP - di of query half mq: acc[r] <-> query 32mq + 8(r/4) + 4g + r%4, key kcol.
+  // S and dP - di (kRagged: dP) of query half mq: acc[r] <-> query 32mq + 8(r/4) + 4g + r%4,
+  // key kcol.
   auto half_scores = [&](int buf, int mq, f32x16& s, f32x16& dp) {
     zero16(s);
     zero16(dp);
@@ -237,6 +240,7 @@ __device__ __forceinline__ void bwd_body(
       s = mfma32(*reinterpret_cast<const bf16x8*>(qrow + 16 * ks), kreg[ks], s);
       dp = mfma32(*reinterpret_cast<const bf16x8*>(grow + 16 * ks), vreg[ks], dp);
     }
+    if (kRagged) return;
     // Lanes g = 1 feed zeros; a multiply by a lane mask (not a branch around
     // the load) keeps the tile in one basic block.
     const float dd = L.dd[buf][32 * mq + c32] * neg_g0;
@@ -253,11 +257,14 @@ __device__ __forceinline__ void bwd_body(
     for (int j = 0; j < 4; ++j) {
       const int qo = 32 * mq + 8 * j + 4 * g;
       const f32x4 st4 = *reinterpret_cast<const f32x4*>(&L.st[buf][qo]);
+      f32x4 dd4 = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (kRagged) dd4 = *reinterpret_cast<const f32x4*>(&L.dd[buf][qo]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 4 * j + i;
         float p, ds;
-        tile_grad<MODE, FAST, BOUNDED, L2N, POLY>(s[r], dp[r], st4[i], clamp, log2n, p, ds);
+        const float dpp = kRagged ? dp[r] - dd4[i] : dp[r];
+        tile_grad<MODE, FAST, BOUNDED, L2N, POLY>(s[r], dpp, st4[i], clamp, log2n, p, ds);
         if (DIAG && q0 + qo + i < kcol) {
           p = 0.0f;
           ds = 0.0f;

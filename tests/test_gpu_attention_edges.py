@@ -210,3 +210,28 @@ def test_ragged_takes_any_variant_pair(guard, fused):
         want = _abi(q, k, v, g, lo if guard else hi)
         for a, b, name in zip(got, want, ("o", "dq", "dk", "dv")):
             assert rel_l2(a, b) <= 1e-2, name       # bf16 weights and outputs
+
+
+@pytest.mark.parametrize("T", [77, 333])
+def test_ragged_di_in_float32(T):
+    """dP - di where both are near 257 and differ by about 0.02, against float64
+    with the kernel's own o: float32 sums of 64 products leave about 5e-5 of the
+    difference and bf16 ds 2e-3 of it. (di as two bf16 values is off by up to
+    0.004, a fifth of it.)"""
+    q, k, v, g = (x.cuda().float() for x in _rand((1, 2, T, 64), 43, dtype="f32"))
+    v = 0.01 * v
+    v[..., 0], v[..., 1] = 256.0, 1.3671875
+    g[..., 2:] *= 0.25
+    g[..., :2] = 1.0
+    leaves = [x.bfloat16().requires_grad_() for x in (q, k, v)]
+    g = g.bfloat16()
+    o = flash_attention(*leaves, block=T, kind="softmax")
+    dq, dk, _ = torch.autograd.grad(o, leaves, g)
+    qd, kd, vd, gd = (x.detach().double() for x in (*leaves, g))
+    qs = (qd / 8.0).bfloat16().double()
+    s = (qs @ kd.transpose(-1, -2)).masked_fill(
+        torch.ones(T, T, device=o.device).triu(1) > 0, -float("inf"))
+    dp, di = gd @ vd.transpose(-1, -2), (gd * o.detach().double()).sum(-1, keepdim=True)
+    ds = torch.softmax(s, -1) * (dp - di)
+    assert rel_l2(dq, ds @ kd / 8.0) <= 1.5e-2
+    assert rel_l2(dk, ds.transpose(-1, -2) @ qs) <= 1.5e-2
