@@ -92,9 +92,9 @@ int32_t check_aligned(const char* who, std::initializer_list<const void*> ptrs) 
   return 0;
 }
 
-// Bytes of the backward's dQ accumulator, which its workspace starts with.
+// Bytes of the backward's dQ sums, which its workspace starts with.
 int64_t acc_bytes(int B, int H, int T, int D) {
-  return (int64_t)B * H * acc_rows(T) * D * (int64_t)sizeof(float);
+  return (int64_t)dq_slots(B, H, T, D) * B * H * acc_rows(T) * D * (int64_t)sizeof(float);
 }
 
 // Row blocks of the backward pre-pass per (b, h), whichever the dtype.
@@ -196,14 +196,11 @@ extern "C" int32_t algx_attn_forward_unit(const void* q, const void* k, const vo
   const bool pair = guard == nullptr || mfma_fused_pair(kl, kh);
   if (use_mfma(T, D, dtype, pair && parts)) {
     if (!parts) return fail("attn_forward: the guard needs the workspace");
-    // The backward workspace starts with its float32 dQ accumulator.
+    // The backward workspace starts with its float32 dQ sums: an accumulator
+    // to clear where T is whole blocks.
     return launch_fwd_fused(q, k, v, sink, q_s, o, o_precise, stat, guard, (float*)workspace,
                             (float*)bwd_workspace, B, H, T, q_scale, bound, vmax, kl, kh, s);
   }
-  // The backward of such a call may still run MFMA and finds its accumulator
-  // cleared.
-  if (bwd_workspace != nullptr && use_mfma(T, D, dtype, mfma_pair(kl, kh)))
-    if (int32_t rc = fill_f32((float*)bwd_workspace, acc_bytes(B, H, T, D) / 4, 0.0f, s)) return rc;
   if (int32_t rc = launch_prepare(q, k, v, sink, q_s, guard, B, H, T, D, dtype, q_scale, bound,
                                   vmax, sink_unit, s))
     return rc;
@@ -268,13 +265,14 @@ extern "C" int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* 
   float* dq_acc = (float*)workspace;
   float* di = (float*)((char*)workspace + acc_bytes(B, H, T, D));
   // The pre-pass forms di and the shares of dsink, and clears the dQ
-  // accumulator unless the forward already did (a workspace it prepared).
-  const bool cleared = mfma && workspace_state == ALGX_ATTN_WS_CLEARED;
+  // accumulator unless the forward already did (a workspace it prepared) or
+  // the key blocks store to slots of their own.
+  const bool clear = mfma && whole_blocks(T) && workspace_state != ALGX_ATTN_WS_CLEARED;
   float* shares = (float*)((char*)di + ((rows * (int64_t)sizeof(float) + 255) / 256) * 256);
   const SinkGrad sg{shares, sink != nullptr ? dsink : nullptr, pre_blocks(T, D, dtype), B, H,
                     sink_unit};
   if (int32_t rc = launch_bwd_pre(dout, o, o_precise, stat, sink, di,
-                                  mfma && !cleared ? dq_acc : nullptr,
+                                  clear ? dq_acc : nullptr,
                                   sg.dsink != nullptr ? shares : nullptr, B, H, T, D, dtype, kl,
                                   kh, guard, s))
     return rc;
@@ -282,8 +280,7 @@ extern "C" int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* 
     if (int32_t rc = launch_bwd_mfma(q, k, v, stat, di, dout, dq_acc, dk, dv, B, H, T, kl, kh,
                                      guard, s))
       return rc;
-    return launch_dq_finish(dq_acc, dq, (int64_t)B * H, T, D, dtype, kl, kh, guard, q_scale, sg,
-                            s);
+    return launch_dq_finish(dq_acc, dq, B, H, T, kl, kh, guard, q_scale, sg, s);
   }
   if (sg.dsink != nullptr)
     if (int32_t rc = launch_sink_finish(sg, s)) return rc;

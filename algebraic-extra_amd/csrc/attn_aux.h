@@ -24,7 +24,7 @@ struct SinkGrad {
 };
 // Row pre-pass of the backward: di (and, with a sink and sink_part, each
 // block's share of the sink gradient, pre_blocks() per (b, h)), and the dQ
-// accumulator cleared when dq_acc is given.
+// accumulator (T in whole 128-row blocks) cleared when dq_acc is given.
 int pre_blocks(int T, int D, int dtype);
 int32_t launch_bwd_pre(const void* dout, const void* o, const float* o_precise,
                        const float* stat, const float* sink, float* di, float* dq_acc,
@@ -33,9 +33,10 @@ int32_t launch_bwd_pre(const void* dout, const void* o, const float* o_precise,
                        hipStream_t s);
 // dsink from the shares, as a launch of its own or in the dQ finish.
 int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s);
-int32_t launch_dq_finish(const float* acc, void* dq, int64_t heads, int T, int D, int dtype,
-                         const KVariant& low, const KVariant& high, const int32_t* guard,
-                         float q_scale, const SinkGrad& sg, hipStream_t s);
+// dq (bf16, D = 64) of the MFMA backward from its float32 sums.
+int32_t launch_dq_finish(const float* acc, void* dq, int B, int H, int T, const KVariant& low,
+                         const KVariant& high, const int32_t* guard, float q_scale,
+                         const SinkGrad& sg, hipStream_t s);
 
 // Generic kernels: any T, D in {16, 32, 64}, bf16 or f32, every variant. With a
 // guard word they run `lo` or `hi` for the whole call, else `lo`.
@@ -57,10 +58,28 @@ bool mfma_supported(int T, int D, int dtype);
 // there; other T have no other kernels and are refused.
 bool mfma_pair(const KVariant& lo, const KVariant& hi);
 bool mfma_fused_pair(const KVariant& lo, const KVariant& hi);
-// Rows per head of the MFMA backward's float32 dQ accumulator: T rounded up to
-// whole 128-row query blocks, so that the forward clears and the backward adds
-// whole blocks.
+// Rows per head of the MFMA backward's float32 dQ sums: T rounded up to whole
+// 128-row query blocks, so that the backward stores whole tiles.
 __host__ __device__ inline int acc_rows(int T) { return (T + 127) / 128 * 128; }
+// Keys of a workgroup of the MFMA backward.
+constexpr int kBwdKeys = 256;
+// Copies (slots) of those sums in the workspace. One where T is a multiple of
+// 128: the key blocks add to it with atomics. Elsewhere dq is the same in every
+// run, as it was on the generic kernels: a launch takes at most this many key
+// blocks, each with a slot of its own, the next launch adds its blocks to the
+// slots, and the finish adds the slots in order. Four at least, else as many as
+// one launch of a workgroup per compute unit takes, so that the slots of a
+// large batch stay at four. The reads of the finish are the price: forward and
+// backward against atomics into one accumulator, B=2, H=12, T=333 95-99 -> 85
+// us, B=8, H=16, T=700 95 -> 93, B=8, H=24, T=1023 211 -> 219, B=8, H=16, T=2047
+// 424 -> 452 us.
+inline int dq_slots(int B, int H, int T, int D) {
+  const int64_t bh = (int64_t)B * H;
+  if (D != 64 || T % 128 == 0 || bh <= 0) return 1;
+  const int64_t nkb = (T + kBwdKeys - 1) / kBwdKeys, fill = (256 + bh - 1) / bh;
+  const int64_t n = fill > 4 ? fill : 4;
+  return (int)(n < nkb ? n : nkb);
+}
 // One launch per call: with a guard word the kernel runs `lo` or `hi` for the
 // whole grid; without one it runs `lo`.
 int32_t launch_fwd_mfma(const void* q_s, const void* k, const void* v, const float* sink,

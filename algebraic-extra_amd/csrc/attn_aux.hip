@@ -193,10 +193,9 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(
       if (has_sink) ds_acc += sink_grad_term(var, b, stat[row], acc);
     }
     if (dq_acc != nullptr) {
-      const int64_t aoff = ((int64_t)bh * acc_rows(T_) + t) * D + sub * EPL;
       f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int i = 0; i < EPL; i += 4) *reinterpret_cast<f32x4*>(dq_acc + aoff + i) = z;
+      for (int i = 0; i < EPL; i += 4) *reinterpret_cast<f32x4*>(dq_acc + off + i) = z;
     }
   }
   if (has_sink && sink_part != nullptr) {
@@ -233,12 +232,9 @@ __global__ __launch_bounds__(256) void sink_finish_kernel(const float* __restric
 
 // dq = cast(cast(acc * slope) * q_scale): the kernel's dQ output rounding
 // (flash.py:592) followed by the VJP of the query pre-scale (flash.py:833).
-// acc holds pad more elements per head of `per_head` than dq does. With a
-// sink, the first sg.H blocks sum its gradient instead (one head each).
-template <typename T>
+// With a sink, the first sg.H blocks sum its gradient instead (one head each).
 __global__ __launch_bounds__(256) void dq_finish_kernel(const float* __restrict__ acc,
-                                                        T* __restrict__ dq, int64_t n,
-                                                        int64_t per_head, int64_t pad,
+                                                        bf16* __restrict__ dq, int64_t n,
                                                         KVariant low, KVariant high,
                                                         const int32_t* __restrict__ guard,
                                                         float q_scale, SinkGrad sg) {
@@ -252,10 +248,42 @@ __global__ __launch_bounds__(256) void dq_finish_kernel(const float* __restrict_
   int64_t i = ((int64_t)(blockIdx.x - nsink) * blockDim.x + threadIdx.x) * 4;
   const int64_t stride = (int64_t)(gridDim.x - nsink) * blockDim.x * 4;
   for (; i < n; i += stride) {
-    const int64_t at = pad != 0 ? i + i / per_head * pad : i;
-    f32x4 a = *reinterpret_cast<const f32x4*>(acc + at);
+    f32x4 a = *reinterpret_cast<const f32x4*>(acc + i);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dq[i + j] = from_f<T>(round_to<T>(a[j] * slope) * q_scale);
+    for (int j = 0; j < 4; ++j) dq[i + j] = from_f<bf16>(round_to<bf16>(a[j] * slope) * q_scale);
+  }
+}
+
+// The same where T is no multiple of 128: row t's sums are those of its key
+// blocks' slots, added in slot order; 16 threads a row.
+__global__ __launch_bounds__(256) void dq_finish_slots_kernel(
+    const float* __restrict__ acc, int slots, bf16* __restrict__ dq, int64_t rows, int T_,
+    KVariant low, KVariant high, const int32_t* __restrict__ guard, float q_scale, SinkGrad sg) {
+  const int nsink = sg.dsink != nullptr ? sg.H : 0;
+  if ((int)blockIdx.x < nsink) {
+    sum_sink(sg.part, sg.nblk, sg.B, sg.H, blockIdx.x, sg.unit, sg.dsink);
+    return;
+  }
+  const KVariant& var = guard_in_range(guard) ? low : high;
+  const float slope = var.slope;
+  const int arows = acc_rows(T_);
+  const int64_t slot = rows / T_ * arows * 64;  // elements of a slot
+  const int d0 = 4 * (threadIdx.x & 15);
+  int64_t row = (int64_t)(blockIdx.x - nsink) * 16 + (threadIdx.x >> 4);
+  for (; row < rows; row += (int64_t)(gridDim.x - nsink) * 16) {
+    const int64_t bh = row / T_;
+    const int t = (int)(row - bh * T_), last = min(t / kBwdKeys, slots - 1);
+    const float* p = acc + (bh * arows + t) * 64 + d0;
+    f32x4 a = *reinterpret_cast<const f32x4*>(p);
+    for (int s = 1; s <= last; ++s) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(p + s * slot);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[j] += b[j];
+    }
+    bf16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = from_f<bf16>(round_to<bf16>(a[j] * slope) * q_scale);
+    *reinterpret_cast<bf16x4*>(dq + row * 64 + d0) = v;
   }
 }
 
@@ -356,21 +384,18 @@ int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s) {
   return check_launch("attn_sink_finish");
 }
 
-int32_t launch_dq_finish(const float* acc, void* dq, int64_t heads, int T, int D, int dtype,
-                         const KVariant& low, const KVariant& high, const int32_t* guard,
-                         float q_scale, const SinkGrad& sg, hipStream_t s) {
-  const int64_t per_head = (int64_t)T * D, n = heads * per_head;
-  const int64_t pad = (int64_t)(acc_rows(T) - T) * D;
+int32_t launch_dq_finish(const float* acc, void* dq, int B, int H, int T, const KVariant& low,
+                         const KVariant& high, const int32_t* guard, float q_scale,
+                         const SinkGrad& sg, hipStream_t s) {
+  const int64_t rows = (int64_t)B * H * T, n = rows * 64;
   int64_t nb = (n / 4 + 255) / 256;
   if (nb > 8192) nb = 8192;
-  if (nb < 1) nb = 1;
   if (sg.dsink != nullptr) nb += sg.H;
-  if (dtype == ALGX_BF16)
-    dq_finish_kernel<bf16><<<(int)nb, 256, 0, s>>>(acc, (bf16*)dq, n, per_head, pad, low, high,
-                                                   guard, q_scale, sg);
+  if (T % 128 == 0)
+    dq_finish_kernel<<<(int)nb, 256, 0, s>>>(acc, (bf16*)dq, n, low, high, guard, q_scale, sg);
   else
-    dq_finish_kernel<float><<<(int)nb, 256, 0, s>>>(acc, (float*)dq, n, per_head, pad, low, high,
-                                                    guard, q_scale, sg);
+    dq_finish_slots_kernel<<<(int)nb, 256, 0, s>>>(acc, dq_slots(B, H, T, 64), (bf16*)dq, rows, T,
+                                                   low, high, guard, q_scale, sg);
   return check_launch("attn_dq_finish");
 }
 

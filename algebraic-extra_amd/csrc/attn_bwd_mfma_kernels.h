@@ -16,7 +16,8 @@
 // forms a 16-query x 32-d block of the tile's dQ over all 256 keys with
 // v_mfma_f32_16x16x32_bf16 (dS through transposing reads, K from a K^T copy
 // in LDS with 16-byte reads) and adds it to a float32 accumulator with
-// no-return atomics: one add per element per 256 keys.
+// no-return atomics: one add per element per 256 keys (into a slot of its own,
+// without atomics, where T is no multiple of 128).
 //
 // Pipelining: Q_s/dO/stat/di tiles and dS^T are double-buffered in LDS, so a
 // tile needs one barrier. The dQ of tile t-1 is formed while tile t's
@@ -25,7 +26,7 @@
 // Included by two translation units: ALGX_ATTN_RAGGED 0 for T a multiple of
 // 128, 1 for any other T. There a row past the end reads row T - 1: such a
 // query's statistic makes its weights zero, such a key lies above the diagonal
-// of every query that counts, and the dQ accumulator has whole 128-row blocks
+// of every query that counts, and the dQ sums have whole 128-row blocks
 // per head, so only the tile loader tests bounds. (One kernel for both cost
 // the B=8, H=16, T=2048 layer about 1 %.) di is subtracted in float32 there, as
 // by the kernels that ran these lengths before, not as two bf16 values: with
@@ -43,7 +44,7 @@ namespace mfma {
 namespace {
 
 constexpr bool kRagged = ALGX_ATTN_RAGGED;
-constexpr int BKN = 256;   // keys per workgroup
+constexpr int BKN = kBwdKeys;  // keys per workgroup
 constexpr int BQ = 64;     // queries per tile
 constexpr int NWAVE = 8;
 constexpr int NTHR = 64 * NWAVE;
@@ -125,6 +126,21 @@ __device__ __forceinline__ void tile_grad(float s, float dpp, float st, float cl
   if (MODE == MODE_NOSHIFT && !BOUNDED && !(s < clamp)) ds = 0.0f;
 }
 
+// Where dQ goes: added to an accumulator over all key blocks, or (kRagged) the
+// key blocks kb0 .. kb0 + nkb - 1 of this launch each to a slot of their own,
+// stored by the first launch and added to by the later ones.
+#if ALGX_ATTN_RAGGED
+struct DqOut {
+  float* acc;
+  int64_t slot;  // elements of a slot
+  int kb0, nkb;
+};
+#else
+struct DqOut {
+  float* acc;
+};
+#endif
+
 struct BwdLds {
   bf16 q[2][BQ * RSTR];     // Q_s tile, row-major [query][d]
   bf16 g[2][BQ * RSTR];     // dO tile
@@ -138,12 +154,22 @@ template <int MODE, bool FAST, bool BOUNDED, int L2N, bool POLY>
 __device__ __forceinline__ void bwd_body(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const float* __restrict__ stat, const float* __restrict__ di, const bf16* __restrict__ dout,
-    float* __restrict__ dq_acc, bf16* __restrict__ dk, bf16* __restrict__ dv, int T_,
+    const DqOut& dqo, bf16* __restrict__ dk, bf16* __restrict__ dv, int T_,
     const KVariant& var, BwdLds& L) {
+#if ALGX_ATTN_RAGGED
+  const int nkb = dqo.nkb;
+#else
   const int nkb = (T_ + BKN - 1) / BKN;
+#endif
   const int nheads = gridDim.x / nkb;
   int bh, kb;
   map_block(blockIdx.x, nheads, nkb, false, bh, kb);
+#if ALGX_ATTN_RAGGED
+  float* const dq_acc = dqo.acc + kb * dqo.slot;
+  kb += dqo.kb0;
+#else
+  float* const dq_acc = dqo.acc;
+#endif
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 5, c32 = lane & 31;
   const int G = lane >> 4, i16 = lane & 15, j4 = i16 >> 2, m4 = i16 & 3;
   const int64_t base = (int64_t)bh * T_ * HD;
@@ -325,11 +351,25 @@ __device__ __forceinline__ void bwd_body(
     }
     // acc[i]: dQ[qt*64 + qr + 4G + i][dc + 16nb + i16]
     float* dst = dq_acc + abase + (int64_t)(qt * BQ + qr + 4 * G) * HD + dc + i16;
+#if ALGX_ATTN_RAGGED
+    if (dqo.kb0 > 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc0[i] += dst[i * HD];
+        acc1[i] += dst[i * HD + 16];
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      dst[i * HD] = acc0[i];
+      dst[i * HD + 16] = acc1[i];
+    }
+#else
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       atomicAdd(dst + (int64_t)i * HD, acc0[i]);
       atomicAdd(dst + (int64_t)i * HD + 16, acc1[i]);
     }
+#endif
   };
 
   // Prologue: every setup load (the wave's K and V rows, the K^T block and
@@ -427,19 +467,18 @@ template <int LO, int HI>
 __global__ __launch_bounds__(NTHR, 1) void bwd_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const float* __restrict__ stat, const float* __restrict__ di, const bf16* __restrict__ dout,
-    float* __restrict__ dq_acc, bf16* __restrict__ dk, bf16* __restrict__ dv, int T_,
-    KVariant lo, KVariant hi, const int32_t* __restrict__ guard) {
+    DqOut dqo, bf16* __restrict__ dk, bf16* __restrict__ dv, int T_, KVariant lo, KVariant hi, const int32_t* __restrict__ guard) {
   __shared__ __attribute__((aligned(16))) BwdLds lds;
   if (LO == HI || guard_in_range(guard))
     bwd_body<cfg_mode(LO), cfg_fast(LO), cfg_bounded(LO), cfg_l2n(LO), cfg_poly(LO)>(
-        q, k, v, stat, di, dout, dq_acc, dk, dv, T_, lo, lds);
+        q, k, v, stat, di, dout, dqo, dk, dv, T_, lo, lds);
   else
     bwd_body<cfg_mode(HI), cfg_fast(HI), cfg_bounded(HI), cfg_l2n(HI), cfg_poly(HI)>(
-        q, k, v, stat, di, dout, dq_acc, dk, dv, T_, hi, lds);
+        q, k, v, stat, di, dout, dqo, dk, dv, T_, hi, lds);
 }
 
 typedef void (*BwdFn)(const bf16*, const bf16*, const bf16*, const float*, const float*,
-                      const bf16*, float*, bf16*, bf16*, int, KVariant, KVariant,
+                      const bf16*, DqOut, bf16*, bf16*, int, KVariant, KVariant,
                       const int32_t*);
 
 BwdFn pick_bwd(int cl, int ch) { ALGX_PICK_ALL(bwd_mfma_kernel) }
@@ -448,13 +487,26 @@ int32_t launch_bwd_as(const void* q, const void* k, const void* v, const float* 
                       const float* di, const void* dout, float* dq_acc, void* dk, void* dv,
                       int B, int H, int T, const KVariant& lo, const KVariant& hi,
                       const int32_t* guard, hipStream_t s) {
-  const int grid = B * H * ((T + BKN - 1) / BKN);
+  const int nkb = (T + BKN - 1) / BKN;
   BwdFn fn = pick_bwd(cfg_for(lo), guard != nullptr ? cfg_for(hi) : cfg_for(lo));
   if (fn == nullptr) return fail("attn_bwd: no MFMA kernel for this variant pair");
-  launch_k(probe_for(ALGX_PROBE_ATTN_BWD), fn, dim3(grid), dim3(NTHR), s, (const bf16*)q,
-           (const bf16*)k, (const bf16*)v, stat, di, (const bf16*)dout, dq_acc, (bf16*)dk,
-           (bf16*)dv, T, lo, hi, guard);
-  return check_launch("attn_bwd_mfma");
+  auto launch = [&](int blocks, const DqOut& dqo) {
+    launch_k(probe_for(ALGX_PROBE_ATTN_BWD), fn, dim3(B * H * blocks), dim3(NTHR), s,
+             (const bf16*)q, (const bf16*)k, (const bf16*)v, stat, di, (const bf16*)dout, dqo,
+             (bf16*)dk, (bf16*)dv, T, lo, hi, guard);
+    return check_launch("attn_bwd_mfma");
+  };
+#if ALGX_ATTN_RAGGED
+  const int slots = dq_slots(B, H, T, HD);
+  const int64_t slot = (int64_t)B * H * acc_rows(T) * HD;
+  for (int kb0 = 0; kb0 < nkb; kb0 += slots) {
+    const int n = slots < nkb - kb0 ? slots : nkb - kb0;
+    if (int32_t rc = launch(n, DqOut{dq_acc, slot, kb0, n})) return rc;
+  }
+  return 0;
+#else
+  return launch(nkb, DqOut{dq_acc});
+#endif
 }
 
 }  // namespace

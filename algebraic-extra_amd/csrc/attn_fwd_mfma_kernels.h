@@ -361,11 +361,10 @@ __device__ __forceinline__ void fwd_body(
     if (g == 0) stat[(int64_t)bh * T_ + qrow] = final_stat(var, m_row, l_tot);
   }
   if (!EARLY_QS) store_prep();
-  if (prep.dq_zero != nullptr) {
-    // The workgroup's 128 query rows of the accumulator (whole blocks of rows
-    // per head) are one contiguous 32 KB run: eight coalesced 16-byte stores
-    // per thread.
-    f32x4* z = reinterpret_cast<f32x4*>(prep.dq_zero + ((int64_t)bh * ntiles * FBM + q0) * HD);
+  if (!kRagged && prep.dq_zero != nullptr) {
+    // The workgroup's 128 query rows of the accumulator are one contiguous
+    // 32 KB run: eight coalesced 16-byte stores per thread.
+    f32x4* z = reinterpret_cast<f32x4*>(prep.dq_zero + base + (int64_t)q0 * HD);
 #pragma unroll
     for (int i = 0; i < FBM * HD / 4 / 256; ++i) z[tid + 256 * i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }

@@ -30,7 +30,8 @@ enum { ALGX_HEAD_CE = 0, ALGX_HEAD_ALG_CE = 1 };
 /* State of the backward workspace handed to algx_attn_bwd: RAW = contents
  * unspecified; CLEARED = the same buffer was passed as bwd_workspace to the
  * algx_attn_forward call whose outputs the backward receives, with no other
- * use in between (its dQ accumulator is then already zero). */
+ * use in between (where the backward adds dQ to an accumulator, bf16 with
+ * D = 64 and T a multiple of 128, it is then already zero). */
 enum { ALGX_ATTN_WS_RAW = 0, ALGX_ATTN_WS_CLEARED = 1 };
 
 /* Numeric variant of the attention kernels; mirrors the numeric fields of the
@@ -200,7 +201,9 @@ int64_t algx_attn_bwd_workspace_bytes(int32_t B, int32_t H, int32_t T, int32_t D
  * (flash.py:721-723) and may be NULL when sink is NULL. workspace_state:
  * ALGX_ATTN_WS_RAW, or ALGX_ATTN_WS_CLEARED for a workspace the forward
  * prepared (see algx_attn_forward), whose dQ accumulator the backward then
- * does not clear again. */
+ * does not clear again. dk, dv and dsink are the same in every run, and so is
+ * dq except for bf16 with D = 64 and T a multiple of 128, whose key blocks add
+ * to it with float32 atomics. */
 int32_t algx_attn_bwd(const void* q_s, const void* k, const void* v, const float* sink,
                       const void* o, const float* o_precise, const float* stat, const void* dout,
                       void* dq, void* dk, void* dv, float* dsink, void* workspace,
