@@ -280,7 +280,8 @@ extern "C" int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* 
     if (int32_t rc = launch_bwd_mfma(q, k, v, stat, di, dout, dq_acc, dk, dv, B, H, T, kl, kh,
                                      guard, s))
       return rc;
-    return launch_dq_finish(dq_acc, dq, B, H, T, kl, kh, guard, q_scale, sg, s);
+    const BwdRows in{(const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)dout, stat, di};
+    return launch_dq_finish(dq_acc, dq, in, B, H, T, kl, kh, guard, q_scale, sg, s);
   }
   if (sg.dsink != nullptr)
     if (int32_t rc = launch_sink_finish(sg, s)) return rc;

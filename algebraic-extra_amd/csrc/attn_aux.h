@@ -34,9 +34,13 @@ int32_t launch_bwd_pre(const void* dout, const void* o, const float* o_precise,
 // dsink from the shares, as a launch of its own or in the dQ finish.
 int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s);
 // dq (bf16, D = 64) of the MFMA backward from its float32 sums.
-int32_t launch_dq_finish(const float* acc, void* dq, int B, int H, int T, const KVariant& low,
-                         const KVariant& high, const int32_t* guard, float q_scale,
-                         const SinkGrad& sg, hipStream_t s);
+struct BwdRows {  // what the backward read, for rows formed again (attn_rows.h)
+  const bf16 *q, *k, *v, *dout;
+  const float *stat, *di;
+};
+int32_t launch_dq_finish(const float* acc, void* dq, const BwdRows& in, int B, int H, int T,
+                         const KVariant& low, const KVariant& high, const int32_t* guard,
+                         float q_scale, const SinkGrad& sg, hipStream_t s);
 
 // Generic kernels: any T, D in {16, 32, 64}, bf16 or f32, every variant. With a
 // guard word they run `lo` or `hi` for the whole call, else `lo`.

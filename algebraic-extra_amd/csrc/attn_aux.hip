@@ -1,6 +1,7 @@
 // Attention side passes: range guard reduction, backward row pre-pass
 // (di, dsink, dQ accumulator clear) and the dQ finishing cast.
 #include "attn_aux.h"
+#include "attn_rows.h"
 
 namespace algx {
 
@@ -255,10 +256,11 @@ __global__ __launch_bounds__(256) void dq_finish_kernel(const float* __restrict_
 }
 
 // The same where T is no multiple of 128: row t's sums are those of its key
-// blocks' slots, added in slot order; 16 threads a row.
+// blocks' slots, added in slot order; 16 lanes a row. A row that is not finite
+// is formed again over its visible keys.
 __global__ __launch_bounds__(256) void dq_finish_slots_kernel(
-    const float* __restrict__ acc, int slots, bf16* __restrict__ dq, int64_t rows, int T_,
-    KVariant low, KVariant high, const int32_t* __restrict__ guard, float q_scale, SinkGrad sg) {
+    const float* __restrict__ acc, int slots, bf16* __restrict__ dq, BwdRows in, int64_t rows,
+    int T_, KVariant low, KVariant high, const int32_t* __restrict__ guard, float q_scale, SinkGrad sg) {
   const int nsink = sg.dsink != nullptr ? sg.H : 0;
   if ((int)blockIdx.x < nsink) {
     sum_sink(sg.part, sg.nblk, sg.B, sg.H, blockIdx.x, sg.unit, sg.dsink);
@@ -268,10 +270,10 @@ __global__ __launch_bounds__(256) void dq_finish_slots_kernel(
   const float slope = var.slope;
   const int arows = acc_rows(T_);
   const int64_t slot = rows / T_ * arows * 64;  // elements of a slot
-  const int d0 = 4 * (threadIdx.x & 15);
-  int64_t row = (int64_t)(blockIdx.x - nsink) * 16 + (threadIdx.x >> 4);
-  for (; row < rows; row += (int64_t)(gridDim.x - nsink) * 16) {
-    const int64_t bh = row / T_;
+  const int lane = threadIdx.x & 63, r = lane >> 4, d0 = 4 * (lane & 15);
+  int64_t row0 = (int64_t)(blockIdx.x - nsink) * 16 + 4 * (threadIdx.x >> 6);  // the wave's four
+  for (; row0 < rows; row0 += (int64_t)(gridDim.x - nsink) * 16) {
+    const int64_t row = min(row0 + r, rows - 1), bh = row / T_;
     const int t = (int)(row - bh * T_), last = min(t / kBwdKeys, slots - 1);
     const float* p = acc + (bh * arows + t) * 64 + d0;
     f32x4 a = *reinterpret_cast<const f32x4*>(p);
@@ -280,10 +282,22 @@ __global__ __launch_bounds__(256) void dq_finish_slots_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) a[j] += b[j];
     }
-    bf16x4 v;
+    const float x = (a[0] * 0.0f + a[1] * 0.0f) + (a[2] * 0.0f + a[3] * 0.0f);
+    const uint64_t bad = __ballot(x != x);
+    if (row0 + r < rows && (bad >> (16 * r) & 0xffff) == 0) {
+      bf16x4 v;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = from_f<bf16>(round_to<bf16>(a[j] * slope) * q_scale);
-    *reinterpret_cast<bf16x4*>(dq + row * 64 + d0) = v;
+      for (int j = 0; j < 4; ++j) v[j] = from_f<bf16>(round_to<bf16>(a[j] * slope) * q_scale);
+      *reinterpret_cast<bf16x4*>(dq + row * 64 + d0) = v;
+    }
+    if (__builtin_expect(bad == 0, 1)) continue;
+    for (int i = 0; i < 4 && row0 + i < rows; ++i) {
+      if ((bad >> (16 * i) & 0xffff) == 0) continue;
+      const int64_t head = (row0 + i) / T_ * T_, at = row0 + i;
+      const float y = row_dq(var, in.q + head * 64, in.k + head * 64, in.v + head * 64,
+                             in.dout + head * 64, in.stat[at], in.di[at], (int)(at - head), lane);
+      dq[at * 64 + lane] = from_f<bf16>(round_to<bf16>(y * slope) * q_scale);
+    }
   }
 }
 
@@ -384,9 +398,9 @@ int32_t launch_sink_finish(const SinkGrad& sg, hipStream_t s) {
   return check_launch("attn_sink_finish");
 }
 
-int32_t launch_dq_finish(const float* acc, void* dq, int B, int H, int T, const KVariant& low,
-                         const KVariant& high, const int32_t* guard, float q_scale,
-                         const SinkGrad& sg, hipStream_t s) {
+int32_t launch_dq_finish(const float* acc, void* dq, const BwdRows& in, int B, int H, int T,
+                         const KVariant& low, const KVariant& high, const int32_t* guard,
+                         float q_scale, const SinkGrad& sg, hipStream_t s) {
   const int64_t rows = (int64_t)B * H * T, n = rows * 64;
   int64_t nb = (n / 4 + 255) / 256;
   if (nb > 8192) nb = 8192;
@@ -394,8 +408,8 @@ int32_t launch_dq_finish(const float* acc, void* dq, int B, int H, int T, const 
   if (T % 128 == 0)
     dq_finish_kernel<<<(int)nb, 256, 0, s>>>(acc, (bf16*)dq, n, low, high, guard, q_scale, sg);
   else
-    dq_finish_slots_kernel<<<(int)nb, 256, 0, s>>>(acc, dq_slots(B, H, T, 64), (bf16*)dq, rows, T,
-                                                   low, high, guard, q_scale, sg);
+    dq_finish_slots_kernel<<<(int)nb, 256, 0, s>>>(acc, dq_slots(B, H, T, 64), (bf16*)dq, in, rows,
+                                                   T, low, high, guard, q_scale, sg);
   return check_launch("attn_dq_finish");
 }
 

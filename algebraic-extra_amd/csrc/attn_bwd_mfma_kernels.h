@@ -27,7 +27,9 @@
 // 128, 1 for any other T. There a row past the end reads row T - 1: such a
 // query's statistic makes its weights zero, such a key lies above the diagonal
 // of every query that counts, and the dQ sums have whole 128-row blocks
-// per head, so only the tile loader tests bounds. (One kernel for both cost
+// per head, so only the tile loader tests bounds. A key whose dk or dv comes
+// out non-finite is formed again over the queries that see it (attn_rows.h),
+// and so is a query's dq in the finish. (One kernel for both cost
 // the B=8, H=16, T=2048 layer about 1 %.) di is subtracted in float32 there, as
 // by the kernels that ran these lengths before, not as two bf16 values: with
 // di near 257 and dP - di near 0.02 the two values left dq 8 % off. At B=2,
@@ -38,6 +40,7 @@
 #include <type_traits>
 
 #include "attn_mfma.h"
+#include "attn_rows.h"
 
 namespace algx {
 namespace mfma {
@@ -445,10 +448,35 @@ __device__ __forceinline__ void bwd_body(
   }
   dq_tile(nqt - 1, (nqt - 1 - qt0) & 1);
 
+  const float slope = var.slope;
+  // Keys with a non-finite value, bit c of key kw + c (x * 0 is NaN for it).
+  unsigned again = 0;
+  if (kRagged) {
+    float t = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        t = __builtin_fmaf(dka[dt][r], 0.0f, t);
+        t = __builtin_fmaf(dva[dt][r], 0.0f, t);
+      }
+    const uint64_t b = __ballot(t != t && kcol < T_);
+    again = (unsigned)b | (unsigned)(b >> 32);
+    const bool mine = again >> c32 & 1;
+    if (__builtin_expect(again != 0, 0))
+      for (; again != 0; again &= again - 1) {
+        const int key = kw + __builtin_ctz(again);
+        float xk, xv;
+        row_dkdv(var, q + base, k + base, v + base, dout + base, stat + rbase, di + rbase, key, T_,
+                 lane, xk, xv);
+        dk[base + (int64_t)key * HD + lane] = (bf16)(xk * slope);
+        dv[base + (int64_t)key * HD + lane] = (bf16)xv;
+      }
+    if (mine) return;
+  }
   if (kRagged ? kcol >= T_ : !wave_keys) return;
   // dka[dt][r]: dK[kcol][32dt + 8(r/4) + 4g + r%4] (before the slope n).
   const int64_t krow = base + (int64_t)kcol * HD;
-  const float slope = var.slope;
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
 #pragma unroll

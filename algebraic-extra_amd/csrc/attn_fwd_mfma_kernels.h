@@ -22,7 +22,8 @@
 // Included by two translation units: ALGX_ATTN_RAGGED 0 for T in whole
 // 128-query blocks, 1 for any other T. There, rows past the end read row T - 1
 // and are not stored; as keys they lie above the diagonal of every stored row,
-// and a repeated row changes none of the guard's maxima. (One kernel for both
+// and a repeated row changes none of the guard's maxima. A row that comes out
+// non-finite is formed again over its visible keys (attn_rows.h). (One kernel for both
 // cost the B=8, H=16, T=2048 layer about 1 %.) A guarded B=2, H=12, T=333
 // forward took 2 x 220 us on the one-thread-per-row kernels these replace
 // there and takes 13.7 us.
@@ -31,6 +32,7 @@
 #include <type_traits>
 
 #include "attn_mfma.h"
+#include "attn_rows.h"
 
 namespace algx {
 namespace mfma {
@@ -344,7 +346,18 @@ __device__ __forceinline__ void fwd_body(
   const float l_tot = l_row + __shfl_xor(l_row, 32, 64);
   const float inv = 1.0f / l_tot;
   const int64_t orow = base + (int64_t)qrow * HD;
-  if (!kRagged || qrow < T_) {
+  // Rows with a non-finite value, bit c of row qw + c (x * 0 is NaN for it).
+  unsigned again = 0;
+  if (kRagged) {
+    float t = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t = __builtin_fmaf(oacc[dt][r] * inv, 0.0f, t);
+    const uint64_t b = __ballot(t != t && qrow < T_);
+    again = (unsigned)b | (unsigned)(b >> 32);
+  }
+  if (!kRagged || (qrow < T_ && !(again >> c32 & 1))) {
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
@@ -358,8 +371,19 @@ __device__ __forceinline__ void fwd_body(
         if (var.precise && o_precise != nullptr)
           *reinterpret_cast<f32x4*>(o_precise + orow + d) = val;
       }
-    if (g == 0) stat[(int64_t)bh * T_ + qrow] = final_stat(var, m_row, l_tot);
   }
+  if (g == 0 && (!kRagged || qrow < T_))
+    stat[(int64_t)bh * T_ + qrow] = final_stat(var, m_row, l_tot);
+  if (kRagged && __builtin_expect(again != 0, 0))
+    for (; again != 0; again &= again - 1) {
+      const int c = __builtin_ctz(again), row = qw + c;
+      const float x = row_forward(var, q + base, prep.q_s != nullptr ? prep.q_scale : 1.0f,
+                                  k + base, v + base, row, from_lane(m_row, c), lane) *
+                      from_lane(inv, c);
+      const int64_t at = base + (int64_t)row * HD + lane;
+      o[at] = (bf16)x;
+      if (var.precise && o_precise != nullptr) o_precise[at] = x;
+    }
   if (!EARLY_QS) store_prep();
   if (!kRagged && prep.dq_zero != nullptr) {
     // The workgroup's 128 query rows of the accumulator are one contiguous

@@ -255,3 +255,41 @@ def test_ragged_dq_is_the_same_in_every_run(B, H, T):
     want = torch.autograd.grad(torch.softmax(s, -1) @ ref[2], ref, g[-1:, -2:].double())
     for a, b, name in zip(runs[0], want, ("dq", "dk", "dv")):
         assert rel_l2(a[-1:, -2:], b) <= 1e-2, name     # bf16 weights and outputs
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
+@pytest.mark.parametrize("T,j", [(40, 21), (333, 200), (333, 332), (700, 300)])
+@pytest.mark.parametrize("kw", [dict(kind="asinh", n=16, c=8.0, shift=False),
+                                dict(kind="asinh", n=16, c=8.0, shift=True, fast_rho=False),
+                                dict(kind="softmax")], ids=["clamped", "shift", "softmax"])
+def test_ragged_non_finite_rows_stay_apart(T, j, kw, value):
+    """A row j of q, k, v or dO that is not finite reaches only what sees it,
+    also where the bf16 MFMA kernels share its tile or its 256-key block with
+    other rows, or read it again in place of rows past the end. The others are
+    those of finite inputs, up to bf16 weights rounded at another maximum."""
+    q, k, v, g = (x.cuda() for x in _rand((1, 2, T, 64), 53))
+
+    def run(**bad):
+        x = dict(q=q, k=k, v=v, g=g)
+        for name in bad:
+            x[name] = x[name].clone()
+            x[name][0, 1, j] = value
+        leaves = [x[n].detach().requires_grad_() for n in "qkv"]
+        o = flash_attention(*leaves, block=T, **kw)
+        return [t.detach()[0] for t in (o, *torch.autograd.grad(o, leaves, x["g"]))]
+
+    want = run()
+    rows = torch.arange(T, device="cuda")
+    before, after, rest = rows < j, rows > j, rows != j
+    # (output, rows that must not change) for each input with the bad row; the
+    # outputs o, dq, dk, dv
+    cases = dict(q=[(0, rest), (1, rest), (2, after), (3, after)], k=[(0, before), (1, before)],
+                 v=[(0, before), (1, before)], g=[(0, rows >= 0), (1, rest), (2, after), (3, after)])
+    for name, checks in cases.items():
+        got = run(**{name: True})
+        for i, keep in checks:
+            assert torch.equal(got[i][0], want[i][0]), (name, i)
+            if keep.any():
+                assert rel_l2(got[i][1][keep], want[i][1][keep]) <= 1e-2, (name, i)
+        if name in "vg":        # (a clamped score is finite)
+            assert not torch.isfinite(got[dict(v=0, g=1)[name]][1, j]).any()
