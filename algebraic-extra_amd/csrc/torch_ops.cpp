@@ -409,6 +409,7 @@ std::tuple<Tensor, Tensor> add_rms_norm(const Tensor& x, const Tensor& r,
 }
 
 Tensor glu_packed(const Tensor& gu, int64_t act, double beta) {
+  TORCH_CHECK_VALUE(gu.size(-1) >= 2, "glu_packed needs a gate and an up column at least");
   on_device(gu, "glu_packed");
   return GluPacked::apply(aligned(gu), act, beta);
 }
@@ -471,6 +472,7 @@ std::tuple<Tensor, Tensor, Tensor> prologue(const Tensor& qkv, const std::option
                                             const std::optional<Tensor>& cos,
                                             const std::optional<Tensor>& sin, int64_t H,
                                             double eps) {
+  TORCH_CHECK_VALUE(H > 0, "attention_prologue needs one head at least");
   on_device(qkv, "attention_prologue");
   const variable_list out = Prologue::apply(qkv.contiguous(), opt(gain32(q_gain)),
                                             opt(gain32(k_gain)), cos, sin, H, eps);

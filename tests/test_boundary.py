@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from algebraic_amd import _lib
-from algebraic_amd.algebraic import alu, alu_glu, rms_norm
+from algebraic_amd.algebraic import alu, alu_glu, glu_packed, rms_norm
 from algebraic_amd.kernels import flash_attention, fused_head, make_variant, qk_rms_norm
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -286,3 +286,14 @@ def test_concat_cast_validation_without_a_gpu():
     assert lib.algx_concat_cast(ctypes.cast(parts, ctypes.c_void_p), ctypes.cast(cols, ctypes.c_void_p),
                                 1, ctypes.c_void_p(64), 2, 0, None) != 0
     assert b"multiples of 4" in lib.algx_last_error()
+
+
+def test_zero_widths_are_refused_without_a_gpu():
+    """Sizes that the operators divide by are refused before the division: an
+    exception, not the end of the process."""
+    from algebraic_amd.kernels.prologue import attention_prologue
+    for dtype in (torch.bfloat16, torch.float32):
+        with pytest.raises(ValueError):
+            glu_packed(_t((4, 0), dtype))
+        with pytest.raises(ValueError):
+            attention_prologue(_t((2, 8, 0), dtype), 0, None, None, None, None)
