@@ -512,6 +512,8 @@ Tensor heads_to_tokens(const Tensor& a) {
 // x^T g in bf16 for x (T, din), g (T, dout): float32 sums of chunks of T added
 // in chunk order.
 Tensor weight_grad(const Tensor& x, const Tensor& g) {
+  TORCH_CHECK_VALUE(x.dim() == 2 && g.dim() == 2 && g.size(0) >= x.size(0),
+                    "weight_grad needs (T, din) inputs and (T, dout) gradients");
   const Tensor x2 = aligned(x), g2 = aligned(g);
   const int64_t T = x2.size(0), din = x2.size(1), dout = g2.size(1);
   Tensor ws = scratch(algx_weight_grad_workspace_bytes(T, din, dout), x2);

@@ -297,3 +297,11 @@ def test_zero_widths_are_refused_without_a_gpu():
             glu_packed(_t((4, 0), dtype))
         with pytest.raises(ValueError):
             attention_prologue(_t((2, 8, 0), dtype), 0, None, None, None, None)
+
+
+def test_weight_grad_shapes_without_a_gpu():
+    """Only matrices, with a gradient row for every input row."""
+    from algebraic_amd.layout import weight_grad
+    for x, g in (((8, 16, 2), (8, 16)), ((8, 16), (8, 16, 1)), ((16,), (8, 16)), ((8, 16), (4, 16))):
+        with pytest.raises(ValueError):
+            weight_grad(_t(x), _t(g))
