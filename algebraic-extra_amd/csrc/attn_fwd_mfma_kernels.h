@@ -126,6 +126,11 @@ __device__ __forceinline__ void fwd_body(
     sq = nan_to_inf(sq + __shfl_xor(sq, 32, 64));
   }
 
+  // The head's queries for rows formed again at the end; the kernels without
+  // EARLY_QS keep the address in vector registers, their scalar ones are taken.
+  unsigned q_lo = (unsigned)(uintptr_t)(q + base);
+  unsigned q_hi = (unsigned)((uintptr_t)(q + base) >> 32);
+  if (kRagged && !EARLY_QS) asm volatile("" : "+v"(q_lo), "+v"(q_hi));
   const bool has_sink = sink != nullptr;
   float m_row, l_row;
   sink_init(var, has_sink, has_sink ? var.sink(sink, h) : 0.0f, m_row, l_row);
@@ -377,9 +382,24 @@ __device__ __forceinline__ void fwd_body(
   if (kRagged && __builtin_expect(again != 0, 0))
     for (; again != 0; again &= again - 1) {
       const int c = __builtin_ctz(again), row = qw + c;
-      const float x = row_forward(var, q + base, prep.q_s != nullptr ? prep.q_scale : 1.0f,
-                                  k + base, v + base, row, from_lane(m_row, c), lane) *
-                      from_lane(inv, c);
+      const float m = from_lane(m_row, c);
+      auto weight = [&](float s) {  // as consume's, at the row's final maximum
+        float rr;
+        if (MODE == MODE_SOFTMAX)
+          return __builtin_amdgcn_exp2f(__builtin_fmaf(s, kLog2e, -(m * kLog2e)));
+        if (MODE == MODE_SHIFT)
+          return s == -__builtin_inff()
+                     ? 0.0f
+                     : powN<L2N>((FAST ? rho_fast(s, rr) : rho_exact(s, rr)) * rho_exact(-m, rr),
+                                 log2n);
+        const float x = BOUNDED ? s : __builtin_fminf(s, var.clamp);
+        return powN<L2N>(POLY ? rho_poly(x, rr) : FAST ? rho_fast(x, rr) : rho_exact(x, rr), log2n);
+      };
+      const bf16* qh = reinterpret_cast<const bf16*>(
+          (uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane(q_hi) << 32 |
+          (unsigned)__builtin_amdgcn_readfirstlane(q_lo));
+      const float x = row_forward(qh, prep.q_s != nullptr ? prep.q_scale : 1.0f, k + base,
+                                  v + base, row, lane, weight) * from_lane(inv, c);
       const int64_t at = base + (int64_t)row * HD + lane;
       o[at] = (bf16)x;
       if (var.precise && o_precise != nullptr) o_precise[at] = x;

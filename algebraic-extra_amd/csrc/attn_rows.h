@@ -30,9 +30,9 @@ __device__ __forceinline__ float row_dot(const bf16* a, float factor, const bf16
   return s;
 }
 
-__device__ __forceinline__ float from_lane(float x, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-}
+// x of a lane (through LDS: a lane read by register may take its index from M0,
+// which is the direct-to-LDS loads' alone).
+__device__ __forceinline__ float from_lane(float x, int lane) { return __shfl(x, lane, 64); }
 
 // acc += sum_j w(lane j) rows[j][lane], j < n.
 __device__ __forceinline__ void row_add(float& acc, float w, const bf16* rows, int n, int lane) {
@@ -41,27 +41,16 @@ __device__ __forceinline__ void row_add(float& acc, float w, const bf16* rows, i
     acc = __builtin_fmaf(from_lane(w, j), (float)rows[j * 64 + lane], acc);
 }
 
-// A score's weight in the forward of a row whose maximum is m.
-__device__ __forceinline__ float row_weight(const KVariant& var, float s, float m) {
-  float r;
-  if (var.kind == ALGX_SOFTMAX)
-    return __builtin_amdgcn_exp2f(__builtin_fmaf(s, kLog2e, -(m * kLog2e)));
-  if (!var.shift)
-    return pow2n(rho_of(var, var.bounded ? s : __builtin_fminf(s, var.clamp), r), var.log2n);
-  if (s == -__builtin_inff()) return 0.0f;
-  return pow2n(rho_var(s, var.fast, r) * rho_exact(-m, r), var.log2n);
-}
-
-// Value `lane` of sum_j p_j v_j over the keys j <= row of one head; q times
-// factor is the pre-scaled query.
-__device__ __forceinline__ float row_forward(const KVariant& var, const bf16* q, float factor,
-                                             const bf16* k, const bf16* v, int row, float m,
-                                             int lane) {
+// Value `lane` of sum_j weight(score j) v_j over the keys j <= row of one head; q
+// times factor is the pre-scaled query.
+template <typename Weight>
+__device__ __forceinline__ float row_forward(const bf16* q, float factor, const bf16* k,
+                                             const bf16* v, int row, int lane, Weight&& weight) {
   float acc = 0.0f;
 #pragma unroll 1
   for (int k0 = 0; k0 <= row; k0 += 64) {
     const int key = min(k0 + lane, row);
-    const float p = row_weight(var, row_dot(q + (int64_t)row * 64, factor, k + (int64_t)key * 64), m);
+    const float p = weight(row_dot(q + (int64_t)row * 64, factor, k + (int64_t)key * 64));
     row_add(acc, (float)(bf16)p, v + (int64_t)k0 * 64, min(64, row - k0 + 1), lane);
   }
   return acc;
