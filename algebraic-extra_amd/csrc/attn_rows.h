@@ -6,7 +6,9 @@
 // an infinity or NaN of that row is NaN. For T that is no multiple of 128 the
 // kernels that came before skipped such rows, so these kernels form a row that
 // came out non-finite again here: it is non-finite by its own inputs, or finite
-// after all. Otherwise it costs a test of the results. The callers mark the
+// after all. Otherwise it costs a test of the results. A row all of whose values
+// are NaN is left at once (inputs of NaN alone at B=8, H=16, T=2047: forward and
+// backward 131 ms without that, 5.5 with). The callers mark the
 // branch unlikely: by its loop depth alone the register allocator would spill
 // the kernels' main loops for it.
 #pragma once
@@ -19,7 +21,7 @@ namespace algx {
 // factor) with the lane's row b.
 __device__ __forceinline__ float row_dot(const bf16* a, float factor, const bf16* b) {
   float s = 0.0f;
-#pragma unroll 1
+#pragma unroll 2
   for (int c = 0; c < 8; ++c) {
     const bf16x8 x = *reinterpret_cast<const bf16x8*>(a + 8 * c);
     const bf16x8 y = *reinterpret_cast<const bf16x8*>(b + 8 * c);
@@ -36,7 +38,7 @@ __device__ __forceinline__ float from_lane(float x, int lane) { return __shfl(x,
 
 // acc += sum_j w(lane j) rows[j][lane], j < n.
 __device__ __forceinline__ void row_add(float& acc, float w, const bf16* rows, int n, int lane) {
-#pragma unroll 1
+#pragma unroll 8
   for (int j = 0; j < n; ++j)
     acc = __builtin_fmaf(from_lane(w, j), (float)rows[j * 64 + lane], acc);
 }
@@ -52,6 +54,7 @@ __device__ __forceinline__ float row_forward(const bf16* q, float factor, const 
     const int key = min(k0 + lane, row);
     const float p = weight(row_dot(q + (int64_t)row * 64, factor, k + (int64_t)key * 64));
     row_add(acc, (float)(bf16)p, v + (int64_t)k0 * 64, min(64, row - k0 + 1), lane);
+    if (__all(acc != acc)) break;
   }
   return acc;
 }
@@ -84,6 +87,7 @@ __device__ __forceinline__ void row_dkdv(const KVariant& var, const bf16* q, con
     row_grad(var, s, dp, stat[i], di[i], p, ds);
     row_add(dv, p, dout + (int64_t)q0 * 64, n, lane);
     row_add(dk, ds, q + (int64_t)q0 * 64, n, lane);
+    if (__all(dk != dk && dv != dv)) break;
   }
 }
 
@@ -100,6 +104,7 @@ __device__ __forceinline__ float row_dq(const KVariant& var, const bf16* q, cons
     float p, ds;
     row_grad(var, s, dp, stat, di, p, ds);
     row_add(acc, ds, k + (int64_t)k0 * 64, min(64, row - k0 + 1), lane);
+    if (__all(acc != acc)) break;
   }
   return acc;
 }
