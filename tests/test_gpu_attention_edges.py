@@ -158,45 +158,52 @@ def test_minus_infinite_scores(D, dtype, kw):
                 assert rel_l2(a[..., 1:], b[..., 1:]) <= (1e-4 if dtype == "f32" else 2e-2), name
 
 
-def _abi(q, k, v, do, lo, hi=None, guard=None, fused=False):
-    """o, dq, dk, dv of the C ABI calls for the given variants: the forward
-    alone on a guard word set by the caller, or (fused) as one call that forms
-    the word (bounds that every input keeps)."""
+def _abi(q, k, v, do, lo, hi=None, guard=None, entry="split", bounds=None):
+    """o, dq, dk, dv of the C ABI calls for the given variants. Forward entry
+    points: "split", prepare and forward, the guard word set by the caller; or
+    one call that forms the word (expected to be `guard`; without `bounds`, by
+    bounds that every input keeps or misses): "fused" with a workspace,
+    "no_workspace" without one, "noalloc"."""
     B, H, T, D = q.shape
     dt, st, p = _lib.dtype_code(q.dtype), _lib.stream(), _lib.ptr
     scale = 1.0 / (8.0 * math.sqrt(D))
+    bound, vmax = bounds or (1e9 if guard else 0.0, 1e9)
     q_s, o, dq, dk, dv = (torch.empty_like(q) for _ in range(5))
     o_precise = torch.empty(q.shape, dtype=torch.float32, device="cuda")
     stat = torch.empty((B, H, T), dtype=torch.float32, device="cuda")
-    ws = torch.empty(_lib.query("algx_attn_forward_workspace_bytes", B, H, T, D),
-                     dtype=torch.uint8, device="cuda")
-    bws = torch.empty(_lib.query("algx_attn_bwd_workspace_bytes", B, H, T, D),
-                      dtype=torch.uint8, device="cuda")
-    word = None
+    # NaN where the backward expects nothing cleared
+    bws = torch.full((_lib.query("algx_attn_bwd_workspace_bytes", B, H, T, D) // 4,),
+                     float("nan"), device="cuda")
+    ws = word = None
+    if entry == "fused":
+        ws = torch.empty(_lib.query("algx_attn_forward_workspace_bytes", B, H, T, D),
+                         dtype=torch.uint8, device="cuda")
     if guard is not None:
         word = torch.zeros(_lib.query("algx_attn_guard_words"), dtype=torch.int32, device="cuda")
-        word[0] = guard
-    if fused:
-        _lib.call("algx_attn_forward", p(q), p(k), p(v), None, p(q_s), p(o), p(o_precise), p(stat),
-                  p(word), p(ws), p(bws), B, H, T, D, dt, scale, 1e9 if guard else 0.0, 1e9, lo,
-                  hi, st)
+        word[0] = guard if entry == "split" else 7
+    outs = (p(q), p(k), p(v), None, p(q_s), p(o), p(o_precise), p(stat), p(word))
+    tail = (p(bws), B, H, T, D, dt, scale, bound, vmax, lo, hi, st)
+    if entry == "noalloc":
+        _lib.call("algx_attn_forward_noalloc", *outs, *tail)
+    elif entry != "split":
+        _lib.call("algx_attn_forward", *outs, p(ws), *tail)
     else:
         _lib.call("algx_attn_prepare", p(q), p(k), p(v), None, p(q_s), None, B, H, T, D, dt, scale,
                   0.0, 0.0, st)
         _lib.call("algx_attn_fwd", p(q_s), p(k), p(v), None, p(o), p(o_precise), p(stat), B, H, T,
                   D, dt, lo, hi, p(word), st)
+    state = _lib.ATTN_WS_RAW if entry == "split" else _lib.ATTN_WS_CLEARED
     _lib.call("algx_attn_bwd", p(q_s), p(k), p(v), None, p(o), p(o_precise), p(stat), p(do), p(dq),
-              p(dk), p(dv), None, p(bws), _lib.ATTN_WS_CLEARED if fused else _lib.ATTN_WS_RAW, B, H,
-              T, D, dt, scale, lo, hi, p(word), st)
+              p(dk), p(dv), None, p(bws), state, B, H, T, D, dt, scale, lo, hi, p(word), st)
     torch.cuda.synchronize()
     if word is not None:
         assert int(word[0]) == guard
     return o, dq, dk, dv
 
 
-@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("entry", ["split", "fused"])
 @pytest.mark.parametrize("guard", [0, 1])
-def test_ragged_takes_any_variant_pair(guard, fused):
+def test_ragged_takes_any_variant_pair(guard, entry):
     """The C ABI's guarded calls pair any two variants at lengths that are no
     multiple of 128: pairs that the MFMA kernels do not have, against the chosen
     variant alone."""
@@ -206,7 +213,7 @@ def test_ragged_takes_any_variant_pair(guard, fused):
     clamped = _c_variant(make_variant("asinh", 16, 8.0, T, shift=False))
     softmax = _c_variant(make_variant("softmax"))
     for lo, hi in ((shift, clamped), (clamped, shift), (softmax, shift)):
-        got = _abi(q, k, v, g, lo, hi, guard, fused)
+        got = _abi(q, k, v, g, lo, hi, guard, entry)
         want = _abi(q, k, v, g, lo if guard else hi)
         for a, b, name in zip(got, want, ("o", "dq", "dk", "dv")):
             assert rel_l2(a, b) <= 1e-2, name       # bf16 weights and outputs
@@ -293,3 +300,34 @@ def test_ragged_non_finite_rows_stay_apart(T, j, kw, value):
                 assert rel_l2(got[i][1][keep], want[i][1][keep]) <= 1e-2, (name, i)
         if name in "vg":        # (a clamped score is finite)
             assert not torch.isfinite(got[dict(v=0, g=1)[name]][1, j]).any()
+
+
+@pytest.mark.parametrize("tail", [False, True], ids=["in_range", "out_of_range"])
+@pytest.mark.parametrize("T", [77, 333, 700])
+def test_ragged_forward_entry_points(T, tail):
+    """A guarded call at a ragged length through each forward of the C ABI, the
+    backward on the workspace that forward was given: the same outputs bit for
+    bit from the MFMA kernels (one call, one call without allocation, prepare
+    and forward on the two-variant kernels), and the oracle's. Without a
+    workspace the generic kernels run the forward."""
+    q, k, v, g = _rand((2, 3, T, 64), 59)
+    if tail:
+        q[:, :, -1] *= 200.0
+        k[:, :, -1] *= 200.0
+    want, _ = _oracle(q, k, v, g, None, "bf16", kind="asinh", n=16, c=8.0, range_guard=True)
+    x = [t.cuda() for t in (q, k, v, g)]
+    var = make_variant("asinh", 16, 8.0, T)
+    lo = _c_variant(var._replace(shift=False, inv_stat=True, bounded_scores=True))
+    hi = _c_variant(var._replace(shift=True, inv_stat=False, fast_rho=False, precise_output=True))
+    bound = min(16.0, var.clamp / 2)
+    bounds = (bound, min(1e8, 1e37 / (T * (2 * bound + 1) ** 16)))
+    guard = 0 if tail else 1
+    first = _abi(*x, lo, hi, guard, "fused", bounds)
+    _check_all(first, want[:4], "bf16")
+    for entry in ("noalloc", "split", "no_workspace"):
+        got = _abi(*x, lo, hi, guard, entry, bounds)
+        for a, b, name in zip(got, first, ("o", "dq", "dk", "dv")):
+            if entry == "no_workspace":
+                assert rel_l2(a, b) <= 1e-2, name       # bf16 weights and outputs
+            else:
+                assert torch.equal(a, b), (entry, name)
