@@ -1,10 +1,11 @@
 // C ABI of the attention kernels: argument validation, variant conversion
 // and dispatch between the MFMA path (bf16, D=64) and the generic path
-// (everything else). A guarded MFMA call launches one kernel that reads
-// the device guard word and runs the low or the high variant for the whole
-// grid; the generic path enqueues both variants and the unselected one
-// returns at once. Either way this mirrors lax.cond(in_range, low, high) of
-// flash.py:853-856 without a host round trip.
+// (everything else). A guarded call's kernel reads the device guard word and
+// runs the low or the high variant for the whole grid, on either path: this
+// mirrors lax.cond(in_range, low, high) of flash.py:853-856 without a host
+// round trip. (The fused MFMA forward runs the low variant with the guard's
+// maxima, then a launch of the high one that returns at once where the range
+// holds.)
 #include <initializer_list>
 #include <cstdlib>
 #include <mutex>

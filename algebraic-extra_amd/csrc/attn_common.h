@@ -1,5 +1,5 @@
 // Attention kernel-side variant and the per-element weight math shared by
-// the generic (scalar) and the MFMA kernels.
+// the generic (float32 MFMA) and the bf16 MFMA kernels.
 #pragma once
 
 #include "common.h"

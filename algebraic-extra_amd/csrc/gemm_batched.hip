@@ -386,7 +386,8 @@ int32_t launch_splitk(const void* A, const void* B, void* C, void* workspace, in
 // chunks, in 32-row stages: the rounds, each with a chunk's stages and about 20
 // stages' worth of filling the ring and storing the slice, and the slices
 // written and read again at about 10 TB/s (a stage is about 0.55 us; the slices
-// mostly stay in the Infinity Cache). Chunks of at least 8 stages. Over 16384
+// mostly stay in the Infinity Cache). All chunks but the last, which takes what
+// is left, have 8 stages or more. Over 16384
 // tokens, with the order above: 1024 x 5376 in 3 chunks (252 workgroups)
 // instead of 2 (168) 205 -> 176 us, 1024 x 3072 in 5 instead of 4 136 -> 120-125,
 // 2688 x 1024 in 5 instead of 4 105 -> 96, 768 x 768 57 -> 38.

@@ -581,9 +581,10 @@ int chunk_tokens(int N, int V) {
 // Deals the dh and dE tiles of a chunk of ntok tokens. `share` is one compute
 // unit's equal part of all k stages. A dh tile runs V / 32 stages, so few
 // tokens leave most of the chip idle behind a handful of long tiles: they are
-// cut into chunks of at most a share (of 16 stages at least: below that the
-// 256 KB a chunk leaves in memory costs more than its products). At
-// N = 1024, d = 384, V = 32768 (8 dh tiles of 1024 stages) the launch took
+// cut into chunks of about a share. 16 stages or more are aimed at (below that
+// the 256 KB a chunk leaves in memory costs more than its products); evened
+// out, the chunks of a loop little longer than that have fewer: 17 stages are
+// cut in 9 and 8, 33 in 11. At N = 1024, d = 384, V = 32768 (8 dh tiles of 1024 stages) the launch took
 // 600 us whole and 72 us in 16 chunks, plus 9 us for adding the slots. With
 // many tokens the last dE tiles would run as a partly filled round of whole
 // tiles: the ones that no longer fit into a share are cut in chunks of at

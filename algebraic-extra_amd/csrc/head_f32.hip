@@ -356,8 +356,8 @@ int nchunks_f32(int N, int V) {
 int64_t vpad_f32(int V) { return ((int64_t)V + FT - 1) / FT * FT; }
 
 // k chunks of a rows x cols product over K: enough workgroups to fill the chip,
-// of at least 256 k each (a chunk's slice, written and read again, costs about
-// what 64 k of its products do).
+// of 256 k or more each but the last, which takes what is left (a chunk's slice,
+// written and read again, costs about what 64 k of its products do).
 int gemm_splits(int rows, int cols, int K) {
   const int64_t tiles = (int64_t)((rows + FT - 1) / FT) * ((cols + FT - 1) / FT);
   int64_t s = tiles > 0 ? kF32Groups / tiles : 1;

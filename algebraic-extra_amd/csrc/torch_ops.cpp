@@ -67,7 +67,6 @@ Tensor gain32(const std::optional<Tensor>& g) {
 std::optional<Tensor> opt(const Tensor& t) {
   return t.defined() ? std::optional<Tensor>(t) : std::nullopt;
 }
-// An optional input's slot in a backward's result: one entry either way.
 int64_t rows_of(const Tensor& x) {
   const int64_t D = x.size(-1);
   return D > 0 ? x.numel() / D : 0;

@@ -184,9 +184,11 @@ int32_t algx_attn_bwd_unit(const void* q, const void* k, const void* v, const fl
  * hipMalloc). Same arguments and results, no workspace: the guard's partial
  * maxima live in a static per-device scratch array of the library (768 KiB,
  * held by each GPU the library runs on until the process ends), so
- * B * H * T / 128 may not exceed 65536 whenever a guard word is given (a
- * larger call returns an error before any other check or launch). Every call on one GPU shares that array: calls that
- * overlap on one GPU (concurrent streams) race. */
+ * B * H * floor(T / 128) may not exceed 65536 whenever a guard word is given
+ * (a larger call returns an error before any launch; one that exceeds it only
+ * by its partial last blocks runs on the generic kernels, without the array).
+ * Every call on one GPU shares that array: calls that overlap on one GPU
+ * (concurrent streams) race. */
 int32_t algx_attn_forward_noalloc(const void* q, const void* k, const void* v, const float* sink,
                                   void* q_s, void* o, float* o_precise, float* stat,
                                   int32_t* guard, void* bwd_workspace, int32_t B, int32_t H,
