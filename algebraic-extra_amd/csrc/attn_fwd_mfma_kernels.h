@@ -352,8 +352,11 @@ __device__ __forceinline__ void fwd_body(
   const float inv = 1.0f / l_tot;
   const int64_t orow = base + (int64_t)qrow * HD;
   // Rows with a non-finite value, bit c of row qw + c (x * 0 is NaN for it).
+  // None in the low launch of a guarded call: in range no value overflows, and
+  // out of range, where most do, the high launch writes every row (B=4, H=12,
+  // T=1000 forward and backward took 4046 us with those rows formed again).
   unsigned again = 0;
-  if (kRagged) {
+  if (kRagged && prep.partial == nullptr) {
     float t = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)

@@ -331,3 +331,25 @@ def test_ragged_forward_entry_points(T, tail):
                 assert rel_l2(a, b) <= 1e-2, name       # bf16 weights and outputs
             else:
                 assert torch.equal(a, b), (entry, name)
+
+
+def test_ragged_out_of_range_forms_no_row_twice():
+    """Out of range the guarded forward's first launch overflows in most rows;
+    the second one writes them all, and the first must not form them again one
+    by one (60 times the time at T = 1000). The fastest of ten forwards against
+    that of the next whole-block length, with room for a busy machine."""
+    times = []
+    for T in (1000, 1024):
+        q, k, v, _ = (x.cuda() for x in _rand((4, 12, T, 64), 61))
+        best = math.inf
+        for _ in range(10):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            o = flash_attention(20.0 * q, 20.0 * k, v, block=T, kind="asinh", n=16, c=8.0,
+                                range_guard=True)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        assert torch.isfinite(o).all()
+        times.append(best)
+    assert times[0] <= 8.0 * times[1], times
