@@ -73,10 +73,11 @@ constexpr int kBwdKeys = 256;
 // blocks, each with a slot of its own, the next launch adds its blocks to the
 // slots, and the finish adds the slots in order. Four at least, else as many as
 // one launch of a workgroup per compute unit takes, so that the slots of a
-// large batch stay at four. The reads of the finish are the price: forward and
-// backward against atomics into one accumulator, B=2, H=12, T=333 95-99 -> 85
-// us, B=8, H=16, T=700 95 -> 93, B=8, H=24, T=1023 211 -> 219, B=8, H=16, T=2047
-// 424 -> 452 us.
+// large batch stay at four. The reads of the finish are the price: all kernels
+// of a guarded forward and backward, against atomics into one accumulator (and
+// di as two bf16 values, no row formed again), B=2, H=12, T=333 54.1 -> 53.2 us,
+// B=8, H=16, T=700 99.8 -> 97.5, B=8, H=24, T=1023 225 -> 239 (finish 13 -> 25),
+// B=8, H=16, T=2047 444 -> 477 us (finish 17 -> 39, backward 289 -> 302).
 inline int dq_slots(int B, int H, int T, int D) {
   const int64_t bh = (int64_t)B * H;
   if (D != 64 || T % 128 == 0 || bh <= 0) return 1;

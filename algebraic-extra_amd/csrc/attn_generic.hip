@@ -25,11 +25,11 @@
 // per wave in flight, a wave loads the next tile's operands before the current
 // tile's products. Measured against the one-thread-per-row kernels these
 // replace (whose chains of D FMAs per score left all but a few CUs idle),
-// float32 guarded calls: forward B=1, H=4, T=256 287 -> 13 us; B=2, H=12, T=512
-// forward 575 -> 33 us, backward 1223 -> 108 us (with a second launch per kernel
-// for the variant the guard does not take, which returned at once; the kernels
-// now choose the variant themselves, and the first call as a whole went from 21
-// to 18 us). The distance from float64 did not grow (5.9e-7 ->
+// float32 guarded calls: B=1, H=4, T=256 forward, a whole call, 285 -> 18 us (its
+// three kernels 15.4, this one 9.4); B=2, H=12, T=512, these kernels alone,
+// forward 575 -> 27 us, dK/dV and dQ 1223 -> 94 us. A guarded call is one launch
+// of each, which chooses the variant: with one launch per variant the first
+// call took 21 us. The distance from float64 did not grow (5.9e-7 ->
 // 5.6e-7 of o at the first shape).
 #include "attn_aux.h"
 

@@ -589,7 +589,8 @@ int chunk_tokens(int N, int V) {
 // many tokens the last dE tiles would run as a partly filled round of whole
 // tiles: the ones that no longer fit into a share are cut in chunks of at
 // least 128 stages (a chunk's slot, written and read again, costs about 25
-// stages): 3116 us whole, 2838 + 7 us so at N = 16384, d = 1024, V = 50304.
+// stages): 3088 us whole, 2778 + 7 us so at N = 16384, V = 50304, d = 1024, and
+// 2185 whole, 2097 + 35 so at d = 768.
 GradPlan grad_plan(int ntok, int d, int V, bool dma) {
   constexpr int kUnits = 256;
   GradPlan pl{};
